@@ -1,7 +1,7 @@
 """Performance cases of the library: the calls a serving program makes, over the sizes it makes them at.
 
 The model shapes are the repository's own: the Qwen2-0.5B decode stack (24 layers, hidden 896, vocab 151936), the
-flow head and aggregator (hidden 1024, 8 blocks) and the VAE decoder (24 layers, hidden 896, n_fft 3528).  Each
+flow head (hidden 1024, 8 blocks) and the VAE decoder (24 layers, hidden 896, n_fft 3528).  Each
 case is a dict with an "op" and its sizes:
 
   decode     one token of the whole 24-layer stack on a contiguous cache of `ctx` rows, 4-bit or bf16 weights,
@@ -11,7 +11,6 @@ case is a dict with an "op" and its sizes:
   batch      one token of each of `n` requests of ragged length (`lo`..`hi` cached rows) through four layers of
              the stack over the paged cache, with the tied head and all logits
   flow       the flow head's ten Euler steps for `n` requests (n = 1: ming_cfm_sample, else the batched call)
-  aggregate  the latent's way back to the next LM input row (once per token)
   vae        the decoder from `T` latents to samples, bf16 or 4-bit weights: short chunks when audio is streamed,
              long ones when an utterance is decoded at once
 
