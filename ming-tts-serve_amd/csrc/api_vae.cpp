@@ -1,6 +1,6 @@
 // C-ABI glue of the VAE decoder (include/ming_hip.h, "VAE decoder";
 // Model.vaeDecode, src/ming_model.zig:1257-1309): the model handle with the
-// ISTFT basis built at load time, and the per-fragment decode.
+// ISTFT tables built at load time, and the per-fragment decode.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,12 +20,19 @@ struct ming_vae_model {
     const uint16_t *fc1_bias = nullptr, *head_bias = nullptr, *norm = nullptr;
     const float* window = nullptr;
     std::vector<ming_lm_layer_w> layers;
-    DevBuf basis;                                     // f32 [n_fft][ldspec]: irfft rows
-    DevBuf lat, y1, xs, h, qkv, att, x1, hh, p, spec, frames, part;  // part: split-K partials
+    // inverse transform: the FFT's passes and (cos, sin) table, or (lengths the passes do not
+    // cover, fft.passes == 0) the irfft basis f32 [n_fft][ldspec] and its spectrum rows
+    VFftPlan fft{};
+    DevBuf tw, basis, spec;
+    DevBuf rope;                                      // f32 [F][32][2] (cos, sin)
+    // h, att, hh: bf16 planes; part: K-slice partials (and fc1's sums)
+    DevBuf lat, xs, h, qkv, att, x1, hh, p, frames, part;
     int last_f = 0;
 };
 
 namespace {
+
+constexpr int kMaxSlices = 8;
 
 int vae_err(ming_ctx* ctx, int st, const std::string& m) { return set_err(ctx, st, "vae: " + m); }
 
@@ -44,30 +51,29 @@ VSeg seg_of(const ming_linear& l, const void* bias, int rope, int& wf) {
     return s;
 }
 
-VGemm gemm(const float* a, int lda, int M, int K, float* y, int ldy) {
-    VGemm g{};
-    g.a = a;
-    g.lda = lda;
-    g.M = M;
-    g.K = K;
-    g.y = y;
-    g.ldy = ldy;
-    g.nseg = 1;
-    g.ks = 1;
-    return g;
+// K slices of a residual projection: the row kernel after it adds the partials
+// either way, so a split costs only their traffic.  Few rows: slices of at most
+// eight waves' chunks (K = 4864: 5), so that no wave loops and N / 16 = 56
+// workgroups become 280.  Many rows: enough 64 x 64 tiles to cover the 256 CUs.
+int split_k(int M, int N, int K) {
+    const int blocks = M <= kV3SmallRows ? (K / 32 + 31) / 32 : 1;
+    if (M <= kV3SmallRows) return std::min(kMaxSlices, K > 1024 ? blocks : 1);
+    if (K <= 1024) return 1;  // 32 x 64 tiles
+    const int tiles = ((N + 63) / 64) * ((M + 63) / 64);
+    int ks = 1;
+    while (2 * ks <= kMaxSlices && tiles * ks < 256) ks *= 2;
+    return ks;
 }
 
-// K slices for a GEMM of N columns: enough 64 x 64 workgroups (with the
-// slices) to cover the 256 CUs, each slice whole stages (and whole affine
-// groups), at most 8.
-int split_k(int M, int N, int K, int wf) {
+// K slices of the basis GEMM: enough 64 x 64 workgroups (with the slices) to cover the 256 CUs.
+int split_basis(int M, int N, int K) {
     const int tiles = ((N + 63) / 64) * ((M + 63) / 64);
-    const int unit = wf == VW_Q4 ? 64 : 32;
-    for (int ks = 1; ks <= 8; ks++)
-        if (K % (unit * ks) == 0 && (tiles * ks >= 256 || ks == 8)) return ks;
     int best = 1;
-    for (int ks = 1; ks <= 8; ks++)
-        if (K % (unit * ks) == 0) best = ks;
+    for (int ks = 1; ks <= kMaxSlices; ks++)
+        if (K % (32 * ks) == 0) {
+            best = ks;
+            if (tiles * ks >= 256) break;
+        }
     return best;
 }
 
@@ -123,33 +129,51 @@ int ming_vae_model_create(ming_ctx* ctx, const ming_vae_cfg* cfg, const ming_vae
     m->window = static_cast<const float*>(w->window);
     m->layers.assign(w->layers, w->layers + cfg->n_layers);
     const int N = cfg->n_fft, nb = N / 2 + 1;
-    m->ldspec = (2 * nb + 31) / 32 * 32;
-    // irfft (backward norm) as rows of a matrix: frame[n] = sum_k spec[k] basis[n][k] with
-    // spec = [re_0 .. re_{nb-1} | im_0 .. im_{nb-1} | 0 pad]; bins 1 .. N/2-1 count twice and
-    // the imaginary parts of bins 0 and N/2 are ignored (evaluated in double, rounded once).
-    std::vector<float> basis((size_t)N * m->ldspec, 0.0f);
-    for (int n = 0; n < N; n++) {
-        float* row = basis.data() + (size_t)n * m->ldspec;
-        for (int k = 0; k < nb; k++) {
-            const double c = (k == 0 || 2 * k == N) ? 1.0 : 2.0;
-            const double th = 2.0 * M_PI * (double)(((int64_t)k * n) % N) / (double)N;
-            row[k] = (float)(c * std::cos(th) / N);
-            row[nb + k] = (k == 0 || 2 * k == N) ? 0.0f : (float)(-c * std::sin(th) / N);
-        }
-    }
     const size_t F = (size_t)max_latents * cfg->patch, nq = H + 2 * kvd;
-    hipError_t e = m->basis.ensure(basis.size() * sizeof(float));
-    if (e == hipSuccess)
-        e = hipMemcpy(m->basis.p, basis.data(), basis.size() * sizeof(float), hipMemcpyHostToDevice);
-    const std::pair<DevBuf*, size_t> bufs[] = {
-        {&m->lat, (size_t)max_latents * cfg->latent}, {&m->y1, (size_t)max_latents * H},
-        {&m->xs, (cfg->n_layers + 1) * F * H},        {&m->h, F * H},
-        {&m->qkv, F * nq},                            {&m->att, F * H},
-        {&m->x1, F * H},                              {&m->hh, F * I},
-        {&m->p, F * P},                               {&m->spec, F * m->ldspec},
-        {&m->frames, F * N},                          {&m->part, 8 * F * std::max(nq, (size_t)P)}};
+    std::vector<float> tab;  // evaluated in double, rounded once
+    hipError_t e;
+    if (vfft_plan(N, m->fft)) {
+        tab.resize(2 * (size_t)N);
+        for (int k = 0; k < N; k++) {
+            const double th = 2.0 * M_PI * k / N;
+            tab[2 * k] = (float)std::cos(th);
+            tab[2 * k + 1] = (float)std::sin(th);
+        }
+        e = m->tw.ensure(tab.size() * sizeof(float));
+        if (e == hipSuccess) e = hipMemcpy(m->tw.p, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice);
+    } else {
+        m->fft = VFftPlan{};
+        m->ldspec = (2 * nb + 31) / 32 * 32;
+        // irfft (backward norm) as rows of a matrix: frame[n] = sum_k spec[k] basis[n][k] with
+        // spec = [re_0 .. re_{nb-1} | im_0 .. im_{nb-1} | 0 pad]; bins 1 .. N/2-1 count twice and
+        // the imaginary parts of bins 0 and N/2 are ignored
+        tab.assign((size_t)N * m->ldspec, 0.0f);
+        for (int n = 0; n < N; n++) {
+            float* row = tab.data() + (size_t)n * m->ldspec;
+            for (int k = 0; k < nb; k++) {
+                const double c = (k == 0 || 2 * k == N) ? 1.0 : 2.0;
+                const double th = 2.0 * M_PI * (double)(((int64_t)k * n) % N) / (double)N;
+                row[k] = (float)(c * std::cos(th) / N);
+                row[nb + k] = (k == 0 || 2 * k == N) ? 0.0f : (float)(-c * std::sin(th) / N);
+            }
+        }
+        e = m->basis.ensure(tab.size() * sizeof(float));
+        if (e == hipSuccess) e = hipMemcpy(m->basis.p, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = m->spec.ensure(F * m->ldspec * sizeof(float));
+    }
+    const size_t part_cols = m->ldspec ? std::max((size_t)H, (size_t)N) : (size_t)H;
+    const std::pair<DevBuf*, size_t> bufs[] = {  // bytes
+        {&m->lat, (size_t)max_latents * cfg->latent * 2}, {&m->xs, (cfg->n_layers + 1) * F * H * 4},
+        {&m->h, 3 * F * H * 2},                           {&m->qkv, F * nq * 4},
+        {&m->att, 3 * F * H * 2},                         {&m->x1, F * H * 4},
+        {&m->hh, 3 * F * I * 2},                          {&m->p, F * P * 4},
+        {&m->frames, F * N * 4},                          {&m->part, kMaxSlices * F * part_cols * 4},
+        {&m->rope, F * 64 * 4}};
     for (const auto& b : bufs)
-        if (e == hipSuccess) e = b.first->ensure(b.second * sizeof(float));
+        if (e == hipSuccess) e = b.first->ensure(b.second);
+    if (e == hipSuccess)
+        e = launch_rope_table(ctx->stream, static_cast<float*>(m->rope.p), (int)F, 32, cfg->log2_theta);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
         ming_vae_model_destroy(m);
         return hip_check(ctx, e, "vae workspace");
@@ -160,8 +184,8 @@ int ming_vae_model_create(ming_ctx* ctx, const ming_vae_cfg* cfg, const ming_vae
 
 int ming_vae_model_destroy(ming_vae_model* m) {
     if (!m) return MING_E_NOT_INIT;
-    for (DevBuf* b : {&m->basis, &m->lat, &m->y1, &m->xs, &m->h, &m->qkv, &m->att, &m->x1, &m->hh, &m->p, &m->spec,
-                      &m->frames, &m->part})
+    for (DevBuf* b : {&m->tw, &m->basis, &m->spec, &m->rope, &m->lat, &m->xs, &m->h, &m->qkv, &m->att, &m->x1, &m->hh,
+                      &m->p, &m->frames, &m->part})
         b->release();
     delete m;
     return MING_OK;
@@ -176,79 +200,111 @@ int ming_vae_decode(ming_ctx* ctx, ming_vae_model* m, int32_t T, const void* lat
     const int H = c.hidden, kvd = c.kv_heads * c.head_dim, I = c.inter, nq = H + 2 * kvd, P = c.n_fft + 2;
     const int F = T * c.patch;
     hipStream_t st = ctx->stream;
-    float* xs = static_cast<float*>(m->xs.p);
-    float *h = static_cast<float*>(m->h.p), *qkv = static_cast<float*>(m->qkv.p), *att = static_cast<float*>(m->att.p);
-    float *x1 = static_cast<float*>(m->x1.p), *hh = static_cast<float*>(m->hh.p);
-    hipError_t e = launch_vwiden(st, static_cast<const uint16_t*>(latents), (int64_t)T * c.latent,
-                                 static_cast<float*>(m->lat.p));
+    float *xs = static_cast<float*>(m->xs.p), *qkv = static_cast<float*>(m->qkv.p), *x1 = static_cast<float*>(m->x1.p);
     float* part = static_cast<float*>(m->part.p);
-    // one GEMM: split K where the columns alone leave CUs idle
-    auto run = [&](VGemm g, int wf, int epi, int N) {
-        g.ks = epi == VE_SWIGLU ? 1 : split_k(g.M, N, g.K, wf);
-        g.part = part;
-        return launch_vgemm(st, g, wf, epi);
-    };
+    uint16_t *h = static_cast<uint16_t*>(m->h.p), *att = static_cast<uint16_t*>(m->att.p);
+    uint16_t* hh = static_cast<uint16_t*>(m->hh.p);
+    hipError_t e = hipSuccess;
     int wf = 0;
-    if (e == hipSuccess) {  // fc1: bias and the bf16 rounding are applied by the upsample kernel
-        VGemm g = gemm(static_cast<float*>(m->lat.p), c.latent, T, c.latent, static_cast<float*>(m->y1.p), H);
+    auto gemm = [&](const uint16_t* a, int M, int K, float* y, int ldy) {
+        V3Gemm g{};
+        g.a = a;
+        g.aps = (size_t)M * K;
+        g.np = 3;
+        g.M = M;
+        g.K = K;
+        g.y = y;
+        g.ldy = ldy;
+        g.nseg = 1;
+        g.ks = 1;
+        g.rope_cs = static_cast<const float*>(m->rope.p);
+        return g;
+    };
+    {  // fc1 on the bf16 latents: bias and the bf16 rounding are applied by the row kernel
+        const void* lat = latents;
+        if (reinterpret_cast<uintptr_t>(latents) % 16) {  // the GEMM reads 16-byte words
+            lat = m->lat.p;
+            e = hipMemcpyAsync(m->lat.p, latents, (size_t)T * c.latent * 2, hipMemcpyDeviceToDevice, st);
+        }
+        V3Gemm g = gemm(static_cast<const uint16_t*>(lat), T, c.latent, part, H);
+        g.np = 1;
         g.seg[0] = seg_of(m->fc1, nullptr, 0, wf);
-        e = run(g, wf, VE_PLAIN, H);
+        if (e == hipSuccess) e = launch_v3gemm(st, g, wf, VE_PLAIN);
     }
-    if (e == hipSuccess)
-        e = launch_vup(st, static_cast<float*>(m->y1.p), m->fc1_bias, wf == VW_Q4, T, H, c.patch, xs);
+    // x = (res + the partials) or the upsampled rows, and h = rms_norm(x) for the next linear
+    auto row = [&](const float* res, float* x, int ks, const void* norm, bool up) {
+        VRowArgs a{};
+        a.part = part;
+        a.ks = ks;
+        a.res = res;
+        a.x = x;
+        a.M = F;
+        a.N = H;
+        a.w = static_cast<const uint16_t*>(norm);
+        a.eps = c.eps;
+        a.h = h;
+        a.hps = (size_t)F * H;
+        a.bias = m->fc1_bias;
+        a.q4 = wf == VW_Q4;
+        a.T = T;
+        a.scale = c.patch;
+        return launch_vrow(st, a, up);
+    };
+    if (e == hipSuccess) e = row(nullptr, xs, 0, m->layers[0].ln1, true);
     const float scale = 1.0f / std::sqrt((float)c.head_dim);
+    const int ks_o = split_k(F, H, H), ks_d = split_k(F, H, I);
     for (int l = 0; l < c.n_layers && e == hipSuccess; l++) {
         const ming_lm_layer_w& L = m->layers[l];
         float* x = xs + (size_t)l * F * H;
         float* xo = xs + (size_t)(l + 1) * F * H;
-        e = launch_vrms(st, x, F, H, static_cast<const uint16_t*>(L.ln1), c.eps, h);
-        if (e == hipSuccess) {  // q | k | v in one launch, rotary on q and k
-            VGemm g = gemm(h, H, F, H, qkv, nq);
+        {  // q | k | v in one launch, rotary on q and k
+            V3Gemm g = gemm(h, F, H, qkv, nq);
             g.seg[0] = seg_of(L.wq, L.bq, 1, wf);
             g.seg[1] = seg_of(L.wk, L.bk, 1, wf);
             g.seg[2] = seg_of(L.wv, L.bv, 0, wf);
             g.nseg = 3;
-            g.log2_theta = c.log2_theta;
-            e = run(g, wf, VE_QKV, nq);
+            e = launch_v3gemm(st, g, wf, VE_QKV);
         }
-        if (e == hipSuccess) e = launch_vattn(st, qkv, F, nq, H, c.heads, c.kv_heads, c.window, scale, att);
+        if (e == hipSuccess)
+            e = launch_vattn(st, qkv, F, nq, H, c.heads, c.kv_heads, c.window, scale, att, (size_t)F * H);
         if (e == hipSuccess) {
-            VGemm g = gemm(att, H, F, H, x1, H);
+            V3Gemm g = gemm(att, F, H, part, H);
             g.seg[0] = seg_of(L.wo, nullptr, 0, wf);
-            g.res = x;
-            g.ldres = H;
-            e = run(g, wf, VE_RES, H);
+            g.ks = ks_o;
+            e = launch_v3gemm(st, g, wf, VE_RES);
         }
-        if (e == hipSuccess) e = launch_vrms(st, x1, F, H, static_cast<const uint16_t*>(L.ln2), c.eps, h);
+        if (e == hipSuccess) e = row(x, x1, ks_o, L.ln2, false);
         if (e == hipSuccess) {
-            VGemm g = gemm(h, H, F, H, hh, I);
+            V3Gemm g = gemm(h, F, H, nullptr, 0);
             g.seg[0] = seg_of(L.wg, nullptr, 0, wf);
             g.up = seg_of(L.wu, nullptr, 0, wf);
-            e = run(g, wf, VE_SWIGLU, I);
+            g.yp = hh;
+            g.yps = (size_t)F * I;
+            g.ldyp = I;
+            e = launch_v3gemm(st, g, wf, VE_SWIGLU);
         }
         if (e == hipSuccess) {
-            VGemm g = gemm(hh, I, F, I, xo, H);
+            V3Gemm g = gemm(hh, F, I, part, H);
             g.seg[0] = seg_of(L.wd, nullptr, 0, wf);
-            g.res = x1;
-            g.ldres = H;
-            e = run(g, wf, VE_RES, H);
+            g.ks = ks_d;
+            e = launch_v3gemm(st, g, wf, VE_RES);
         }
+        if (e == hipSuccess) e = row(x1, xo, ks_d, l + 1 < c.n_layers ? m->layers[l + 1].ln1 : m->norm, false);
     }
-    float* p = static_cast<float*>(m->p.p);
-    if (e == hipSuccess) e = launch_vrms(st, xs + (size_t)c.n_layers * F * H, F, H, m->norm, c.eps, h);
+    float *p = static_cast<float*>(m->p.p), *frames = static_cast<float*>(m->frames.p);
     if (e == hipSuccess) {
-        VGemm g = gemm(h, H, F, H, p, P);
+        V3Gemm g = gemm(h, F, H, p, P);
         g.seg[0] = seg_of(m->head, m->head_bias, 0, wf);
-        e = run(g, wf, VE_PLAIN, P);
+        e = launch_v3gemm(st, g, wf, VE_PLAIN);
     }
-    float* spec = static_cast<float*>(m->spec.p);
-    float* frames = static_cast<float*>(m->frames.p);
-    if (e == hipSuccess) e = launch_vspec(st, p, F, c.n_fft, m->ldspec, spec);
-    if (e == hipSuccess) {
-        VGemm g = gemm(spec, m->ldspec, F, m->ldspec, frames, c.n_fft);
-        g.seg[0] = VSeg{m->basis.p, nullptr, nullptr, 1.0f, nullptr, c.n_fft, 0};
-        g.win = m->window;
-        e = run(g, VW_F32, VE_WIN, c.n_fft);
+    if (e == hipSuccess && m->fft.passes) {
+        e = launch_virfft(st, m->fft, p, F, static_cast<const float*>(m->tw.p), m->window, frames);
+    } else if (e == hipSuccess) {
+        float* spec = static_cast<float*>(m->spec.p);
+        e = launch_vspec(st, p, F, c.n_fft, m->ldspec, spec);
+        const VBasis g{spec,   static_cast<const float*>(m->basis.p), F, m->ldspec, c.n_fft, m->window, frames,
+                       split_basis(F, c.n_fft, m->ldspec), part};
+        if (e == hipSuccess) e = launch_vbasis(st, g);
     }
     if (e == hipSuccess) e = launch_vola(st, frames, F, c.n_fft, c.hop, m->window, wave_out);
     if (e == hipSuccess) m->last_f = F;

@@ -119,44 +119,79 @@ constexpr int kImgSlots = 5;  // q/k/v, o_proj, gate/up, down, LM head
 
 constexpr int kMaxParts = 4096;
 
-// ---- VAE decoder GEMM (vae.hip) ----------------------------------------------
-// Weight formats and epilogues of the f32 GEMM.
-enum VWf : int { VW_BF16 = 0, VW_Q4 = 1, VW_F32 = 2 };
+// ---- VAE decoder (vae_gemm.hip, vae.hip) ----
+enum VWf : int { VW_BF16 = 0, VW_Q4 = 1 };
 enum VEpi : int {
     VE_PLAIN = 0,   // y = acc (+ bias)
-    VE_QKV = 1,     // y = acc + bias, rope on columns < rope_cols (heads of 64, position = row)
-    VE_RES = 2,     // y = res + acc
-    VE_SWIGLU = 3,  // y = (g * sigmoid(g)) * u, g from w0, u from w1
-    VE_WIN = 4,     // y = acc * win[col]
+    VE_QKV = 1,     // y = acc + bias, rotary on the segments that ask for it (heads of 64, position = row)
+    VE_RES = 2,     // y [ks][M][ldy] = the K slices' sums (launch_vrow adds them to the residual)
+    VE_SWIGLU = 3,  // planes yp = (g * sigmoid(g)) * u, g from seg[0], u from up
 };
 
-// One weight of the f32 GEMM: bf16 [n][K], MLX affine 4-bit (u32 [n][K/8] +
-// bf16 scales/biases [n][K/64]) or f32 [n][K].
+// One weight of the decoder's linears: bf16 [n][K] or MLX affine 4-bit (u32
+// [n][K/8] + bf16 scales/biases [n][K/64]).
 struct VSeg {
     const void* w;
     const uint16_t *s, *b;
     float gs;               // affine global scale
     const uint16_t* bias;   // bf16 [n] or null (VE_PLAIN, VE_QKV)
     int n;                  // output columns (a multiple of 64 except in the last segment)
-    int rope;               // VE_QKV: 1 = rotary on these columns (heads of 64, position = row)
+    int rope;               // VE_QKV: 1 = rotary on these columns
 };
 
-// C [M][N] = A [M][K] (f32) x W^T; the output columns are the segments'
-// columns one after another (N = sum of seg[i].n).  ks > 1 splits K into ks
-// slices whose partials [ks][M][N] (f32, in part) a reduce kernel sums in
-// slice order before the epilogue.
-struct VGemm {
-    const float* a;
-    int lda, M, K;
+// C [M][N] = A [M][K] x W^T in f32; the output columns are the segments'
+// columns one after another (N = sum of seg[i].n).
+constexpr int kV3SmallRows = 64;  // rows up to which the unstaged kernel runs
+struct V3Gemm {
+    const uint16_t* a;      // bf16 planes [np][M][K] whose sum is A (np = 3, or 1 for a bf16 input)
+    size_t aps;             // values between planes
+    int np, M, K;
     VSeg seg[3];
     int nseg;
-    VSeg up;                // VE_SWIGLU: the up weight over seg[0]'s columns
-    const float* res;       // VE_RES: f32 [M][ldres]
-    int ldres;
-    const float* win;       // VE_WIN: f32 [N]
+    VSeg up;                // VE_SWIGLU
     float* y;
     int ldy;
-    float log2_theta;
+    uint16_t* yp;           // VE_SWIGLU: bf16 planes [3][M][ldyp]
+    size_t yps;
+    int ldyp;
+    const float* rope_cs;   // VE_QKV: f32 [rows][32][2] (cos, sin)
+    int ks;                 // VE_RES: K slices
+};
+
+// The rows between the decoder's linears (launch_vrow): x = res + sum of the K
+// slices part [ks][M][N], or the upsampled rows of the fc1 sums part [T][N]
+// (+ bias, rounded to bf16); h = planes of rms_norm(x) with weight w.
+struct VRowArgs {
+    const float* part;
+    int ks;
+    const float* res;       // f32 [M][N]
+    float* x;               // f32 [M][N]
+    int M, N;
+    const uint16_t* w;      // bf16 [N]
+    float eps;
+    uint16_t* h;            // bf16 [3][M][N]
+    size_t hps;
+    const uint16_t* bias;   // upsample: fc1's bias (bf16 [N] or null), format, latents, factor
+    int q4, T, scale;
+};
+
+// Inverse real FFT of n = 2 h points per frame by passes of the given radices
+// over h complex points (launch_virfft).
+constexpr int kFftMaxHalf = 4096, kFftMaxPasses = 12;
+struct VFftPlan {
+    int h, passes;
+    int radix[kFftMaxPasses];
+};
+
+// C [M][n] = A [M][K] (f32) x W^T (f32 [n][K]) * win[col], for the transforms
+// whose length has a prime factor above 7.  ks > 1 splits K into ks slices whose
+// partials [ks][M][n] a reduce kernel sums in slice order.
+struct VBasis {
+    const float* a;
+    const float* w;
+    int M, K, n;
+    const float* win;
+    float* y;
     int ks;
     float* part;
 };

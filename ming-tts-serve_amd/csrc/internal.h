@@ -137,13 +137,18 @@ struct LmView {
 };
 bool lm_model_view(const ming_lm_model* m, LmView& v);
 
-// ---- VAE decoder (vae.hip) ----
-hipError_t launch_vgemm(hipStream_t st, const VGemm& g, int wf, int epi);
-hipError_t launch_vrms(hipStream_t st, const float* x, int M, int K, const uint16_t* w, float eps, float* out);
+// ---- VAE decoder (vae_gemm.hip, vae.hip) ----
+hipError_t launch_v3gemm(hipStream_t st, const V3Gemm& g, int wf, int epi);
+hipError_t launch_vrow(hipStream_t st, const VRowArgs& a, bool upsample);
 hipError_t launch_vattn(hipStream_t st, const float* qkv, int M, int ldq, int H, int heads, int kvh, int window,
-                        float scale, float* att);
-hipError_t launch_vup(hipStream_t st, const float* y, const uint16_t* bias, int q4, int T, int C, int scale,
-                      float* x);
+                        float scale, uint16_t* att, size_t aps);
+// The passes for an n_fft-point inverse real FFT; false when n_fft / 2 has a
+// prime factor above 7 or does not fit the kernel's LDS.
+bool vfft_plan(int n_fft, VFftPlan& p);
+// tw: (cos, sin)(2 pi k / n_fft), k = 0 .. n_fft - 1
+hipError_t launch_virfft(hipStream_t st, const VFftPlan& pl, const float* p, int F, const float* tw, const float* win,
+                         float* frames);
+hipError_t launch_vbasis(hipStream_t st, const VBasis& g);
 hipError_t launch_vspec(hipStream_t st, const float* p, int F, int nfft, int ld, float* spec);
 hipError_t launch_vola(hipStream_t st, const float* fr, int F, int nfft, int hop, const float* win, float* wave);
 hipError_t launch_vwiden(hipStream_t st, const uint16_t* x, int64_t n, float* y);

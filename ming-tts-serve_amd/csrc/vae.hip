@@ -1,20 +1,111 @@
-// VAE decoder (Model.vaeDecode, src/ming_model.zig:1257-1309): the f32 graph
-// after the latent projection -- linear upsample, the sliding-window Qwen2
-// stack (QStack.forward with window 64, :566-636) and the ISTFT head.
+// VAE decoder, the ISTFT head (Model.vaeDecode, src/ming_model.zig:1257-1309):
+// spectrum, inverse real FFT, synthesis window, overlap-add.  The decoder's
+// linears are in vae_gemm.hip.
 //
-// Every activation after the upsample is f32 in the reference graph (MLX
-// promotes the bf16 weights), so the GEMMs here run on
-// v_mfma_f32_16x16x4f32 with f32 operands: weights are widened exactly (bf16
-// -> f32, MLX affine s*q + b in f32), products are exact and accumulation is
-// f32.  The inverse real FFT is one more GEMM, against an f32 basis of
-// cos/sin rows built at load time, with the synthesis window applied in its
-// epilogue.
+// The inverse transform is an FFT of n_fft / 2 complex points per frame in LDS
+// when n_fft / 2 factors into 2, 3, 5 and 7 (the reference's 3528 = 2 * 1764 =
+// 2 * 7 * 7 * 6 * 6 does), else a GEMM against an f32 basis of cos/sin rows
+// built at load time.
+#include "args.h"
 #include "common.h"
 #include "internal.h"
 
 namespace ming {
 
 namespace {
+
+__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
+    return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
+}
+
+// One Stockham pass of radix R over h points (ns: the product of the radices before it):
+// butterfly b takes src[b + r h / R], turns them by e^{2 pi i (b % ns) r / (ns R)} and writes
+// their R-point transform (sign +) to (b / ns) ns R + b % ns + r ns.
+template <int R>
+__device__ __forceinline__ void fft_pass(const float2* src, float2* dst, int h, int ns, const float2* tw) {
+    const int n = 2 * h, q = h / R, step = n / (ns * R);
+    float2 root[R];
+#pragma unroll
+    for (int k = 1; k < R; k++) root[k] = tw[k * (n / R)];
+    for (int b = threadIdx.x; b < q; b += blockDim.x) {
+        const int k0 = b % ns;
+        float2 v[R], o[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = src[b + r * q];
+#pragma unroll
+        for (int r = 1; r < R; r++) v[r] = cmul(v[r], tw[k0 * r * step]);
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            o[k] = v[0];
+#pragma unroll
+            for (int r = 1; r < R; r++) {
+                if ((k * r) % R == 0) {
+                    o[k].x += v[r].x;
+                    o[k].y += v[r].y;
+                } else {
+                    const float2 w = root[(k * r) % R];
+                    o[k].x = fmaf(v[r].x, w.x, fmaf(-v[r].y, w.y, o[k].x));
+                    o[k].y = fmaf(v[r].x, w.y, fmaf(v[r].y, w.x, o[k].y));
+                }
+            }
+        }
+        float2* d = dst + (b - k0) * R + k0;
+#pragma unroll
+        for (int k = 0; k < R; k++) d[k * ns] = o[k];
+    }
+}
+
+// One workgroup per frame: the head's row p [n_fft + 2] (log-magnitudes | phases) -> windowed
+// time samples.  mag = min(exp(.), 100); the imaginary parts of bins 0 and n_fft / 2 are
+// ignored.  Real output of n = 2 h points from h complex ones: with X the half spectrum,
+// Z[k] = (X[k] + conj X[h - k]) + i e^{2 pi i k / n} (X[k] - conj X[h - k]) has the inverse
+// transform n (x[2 m] + i x[2 m + 1]).
+// Bound: a chain of passes over 2 h values in LDS (n_fft 3528: 28 frames took 38 us and 400
+// frames 145 us as a GEMM against the basis, whose 50 MB alone are 10 us of HBM time).
+__global__ __launch_bounds__(256) void virfft_kernel(VFftPlan pl, const float* __restrict__ p,
+                                                     const float2* __restrict__ tw, const float* __restrict__ win,
+                                                     float* __restrict__ frames) {
+    extern __shared__ float2 fb[];  // two buffers of h
+    const int f = blockIdx.x, h = pl.h, n = 2 * h;
+    const float* pr = p + (size_t)f * (n + 2);
+    float2 *src = fb, *dst = fb + h;
+    auto bin = [&](int k) {
+        const float mag = fminf(expf(pr[k]), 100.0f), ph = pr[h + 1 + k];
+        return make_float2(mag * cosf(ph), k == 0 || k == h ? 0.0f : mag * sinf(ph));
+    };
+    for (int k = threadIdx.x; 2 * k <= h; k += blockDim.x) {
+        const int m = h - k;
+        const float2 a = bin(k), b = bin(m);
+        const float2 e = make_float2(a.x + b.x, a.y - b.y), d = make_float2(a.x - b.x, a.y + b.y);
+        // i e^{i t} d at k; at m the roles swap: conj d -> -conj d, e^{i t} -> -e^{-i t}
+        const float2 t = cmul(d, tw[k]);
+        src[k] = make_float2(e.x - t.y, e.y + t.x);
+        if (k > 0 && m != k) src[m] = make_float2(e.x + t.y, -e.y + t.x);
+    }
+    __syncthreads();
+    int ns = 1;
+    for (int i = 0; i < pl.passes; i++) {
+        switch (pl.radix[i]) {
+            case 2: fft_pass<2>(src, dst, h, ns, tw); break;
+            case 3: fft_pass<3>(src, dst, h, ns, tw); break;
+            case 4: fft_pass<4>(src, dst, h, ns, tw); break;
+            case 5: fft_pass<5>(src, dst, h, ns, tw); break;
+            case 6: fft_pass<6>(src, dst, h, ns, tw); break;
+            default: fft_pass<7>(src, dst, h, ns, tw); break;
+        }
+        ns *= pl.radix[i];
+        __syncthreads();
+        float2* s = src;
+        src = dst;
+        dst = s;
+    }
+    const float inv = 1.0f / (float)n;
+    for (int k = threadIdx.x; k < h; k += blockDim.x) {
+        const float2 v = src[k];
+        *reinterpret_cast<float2*>(frames + (size_t)f * n + 2 * k) =
+            make_float2(v.x * inv * win[2 * k], v.y * inv * win[2 * k + 1]);
+    }
+}
 
 constexpr int kVBM = 64, kVBN = 64, kVBK = 32, kVT = 256;
 constexpr int kVLd = kVBK + 4;  // f32 per LDS row: k permuted so a lane's 8 k-steps are contiguous
@@ -23,145 +114,41 @@ constexpr int kVLd = kVBK + 4;  // f32 per LDS row: k permuted so a lane's 8 k-s
 // so lane group j = lane / 16 reads its 8 values (k-steps kk = 0..7) as two 16-byte words.
 __device__ __forceinline__ int vperm(int k) { return (k & 3) * 8 + (k >> 2); }
 
-struct VTile {  // one thread's share of a stage's global loads
-    float4 a[2];
-    uint4 w[2];    // bf16: w[0] = 8 values; f32: w[0..1] = 8 values as bits; q4: w[0].x = 8 nibbles
-    uint32_t s, b; // q4: scale, bias (bf16 bits)
-};
-
-template <int WF>
-__device__ __forceinline__ void vload_w(const VSeg& sg, int K, int n0, int k0, uint4 (&r)[2], uint32_t& s,
-                                        uint32_t& b) {
-    const int t = threadIdx.x;
-    if (WF == VW_F32) {
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            const int f = t + kVT * p, col = f / 8, kq = f % 8;
-            const int n = min(n0 + col, sg.n - 1);
-            r[p] = ldg4(static_cast<const float*>(sg.w) + (size_t)n * K + k0 + 4 * kq);
-        }
-    } else {
-        const int col = t / 4, kq = t % 4;
-        const int n = min(n0 + col, sg.n - 1);
-        if (WF == VW_BF16) {
-            r[0] = ldg4(static_cast<const uint16_t*>(sg.w) + (size_t)n * K + k0 + 8 * kq);
-        } else {
-            r[0].x = gld(static_cast<const uint32_t*>(sg.w) + (size_t)n * (K / 8) + (k0 + 8 * kq) / 8);
-            s = gld(sg.s + (size_t)n * (K / 64) + (k0 + 8 * kq) / 64);
-            b = gld(sg.b + (size_t)n * (K / 64) + (k0 + 8 * kq) / 64);
-        }
-    }
-}
-
-template <int WF>
-__device__ __forceinline__ void vstore_w(float* lw, const uint4 (&r)[2], uint32_t s, uint32_t b, float gscale) {
-    const int t = threadIdx.x;
-    if (WF == VW_F32) {
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            const int f = t + kVT * p, col = f / 8, kq = f % 8;
-            const uint32_t e[4] = {r[p].x, r[p].y, r[p].z, r[p].w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) lw[col * kVLd + vperm(4 * kq + i)] = __uint_as_float(e[i]);
-        }
-    } else {
-        const int col = t / 4, kq = t % 4;
-        float v[8];
-        if (WF == VW_BF16) {
-            const uint32_t e[4] = {r[0].x, r[0].y, r[0].z, r[0].w};
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                v[2 * i] = bf_lo(e[i]);
-                v[2 * i + 1] = bf_hi(e[i]);
-            }
-        } else {  // MLX affine: s * q + b in f32 (times the global scale)
-            const float fs = bf2f((uint16_t)s), fb = bf2f((uint16_t)b);
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                v[i] = fs * (float)((r[0].x >> (4 * i)) & 15u) + fb;
-                if (gscale != 1.0f) v[i] *= gscale;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) lw[col * kVLd + vperm(8 * kq + i)] = v[i];
-    }
-}
-
-__device__ __forceinline__ int vtotal_n(const VGemm& g) {
-    return g.seg[0].n + (g.nseg > 1 ? g.seg[1].n : 0) + (g.nseg > 2 ? g.seg[2].n : 0);
-}
-
-// The segment holding output column c (segments start at multiples of 64) and its first column.
-__device__ __forceinline__ int vseg_of(const VGemm& g, int c, int& start) {
-    start = 0;
-    int i = 0;
-    while (i + 1 < g.nseg && c >= start + g.seg[i].n) {
-        start += g.seg[i].n;
-        i++;
-    }
-    return i;
-}
-
-// MLX fast::rope of the pair (d, d + 32) of a 64-column head at position `row`.
-__device__ __forceinline__ void vrope(float& x1, float& x2, int d, int row, float log2_theta) {
-    const float inv = exp2f(-((float)d / 32.0f) * log2_theta);
-    const float th = (float)row * inv;
-    const float cs = cosf(th), sn = sinf(th);
-    const float a = x1, b = x2;
-    x1 = a * cs - b * sn;
-    x2 = a * sn + b * cs;
-}
-
-// C [M][N] = A [M][K] (f32, row stride lda) x W^T in format WF; workgroup =
-// 64 x 64 outputs of one segment, wave w = rows 16w .. 16w + 15, all 64
-// columns; K (or its slice blockIdx.z of ks) in stages of 32 through
+// The basis GEMM: workgroup = 64 x 64 outputs, wave w = rows 16w .. 16w + 15, all
+// 64 columns; K (or its slice blockIdx.z of ks) in stages of 32 through
 // double-buffered LDS (the next stage's global loads are in flight during the
-// current stage's MFMAs).  SWIGLU carries the up weight next to the gate.
-// With ks > 1 the raw sums go to the partials and vreduce_kernel applies the
-// epilogue.
-template <int WF, int EPI>
-__global__ __launch_bounds__(kVT) void vgemm_kernel(VGemm g) {
-    constexpr bool DUAL = EPI == VE_SWIGLU;
+// current stage's v_mfma_f32_16x16x4f32).
+__global__ __launch_bounds__(kVT) void vbasis_kernel(VBasis g) {
     __shared__ __align__(16) float la[2][kVBM * kVLd];
     __shared__ __align__(16) float lw[2][kVBN * kVLd];
-    __shared__ __align__(16) float lu[DUAL ? 2 : 1][DUAL ? kVBN * kVLd : 4];
     const int t = threadIdx.x, wave = t / kWave, lane = t % kWave, c = lane % 16, j = lane / 16;
     const int n0 = blockIdx.x * kVBN, m0 = blockIdx.y * kVBM, z = blockIdx.z;
-    const int N = vtotal_n(g);
-    int sstart;
-    const int si = vseg_of(g, n0, sstart);
-    const VSeg& sg = g.seg[si];
-    const int ln0 = n0 - sstart;  // the tile's first column within its segment
     const int Ks = g.K / g.ks, S = Ks / kVBK, kb = z * Ks;
-    VTile r;
-    uint4 ru[2];
-    uint32_t us = 0, ub = 0;
+    float4 ra[2], rw[2];
     auto gload = [&](int s) {
         const int k0 = kb + s * kVBK;
 #pragma unroll
         for (int p = 0; p < 2; p++) {
             const int f = t + kVT * p, row = f / 8, kq = f % 8;
-            r.a[p] = *reinterpret_cast<const float4*>(g.a + (size_t)min(m0 + row, g.M - 1) * g.lda + k0 + 4 * kq);
+            ra[p] = *reinterpret_cast<const float4*>(g.a + (size_t)min(m0 + row, g.M - 1) * g.K + k0 + 4 * kq);
+            rw[p] = *reinterpret_cast<const float4*>(g.w + (size_t)min(n0 + row, g.n - 1) * g.K + k0 + 4 * kq);
         }
-        vload_w<WF>(sg, g.K, ln0, k0, r.w, r.s, r.b);
-        if (DUAL) vload_w<WF>(g.up, g.K, ln0, k0, ru, us, ub);
     };
     auto lstore = [&](int buf) {
 #pragma unroll
         for (int p = 0; p < 2; p++) {
             const int f = t + kVT * p, row = f / 8, kq = f % 8;
-            const float e[4] = {r.a[p].x, r.a[p].y, r.a[p].z, r.a[p].w};
+            const float e[4] = {ra[p].x, ra[p].y, ra[p].z, ra[p].w}, w[4] = {rw[p].x, rw[p].y, rw[p].z, rw[p].w};
 #pragma unroll
-            for (int i = 0; i < 4; i++) la[buf][row * kVLd + vperm(4 * kq + i)] = e[i];
+            for (int i = 0; i < 4; i++) {
+                la[buf][row * kVLd + vperm(4 * kq + i)] = e[i];
+                lw[buf][row * kVLd + vperm(4 * kq + i)] = w[i];
+            }
         }
-        vstore_w<WF>(lw[buf], r.w, r.s, r.b, sg.gs);
-        if (DUAL) vstore_w<WF>(lu[buf], ru, us, ub, g.up.gs);
     };
-    f32x4_t acc[4], accu[DUAL ? 4 : 1];
+    f32x4_t acc[4];
 #pragma unroll
     for (int b = 0; b < 4; b++) acc[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int b = 0; b < (DUAL ? 4 : 1); b++) accu[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     gload(0);
     lstore(0);
     __syncthreads();
@@ -178,212 +165,34 @@ __global__ __launch_bounds__(kVT) void vgemm_kernel(VGemm g) {
             const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
             for (int kk = 0; kk < 8; kk++) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[kk], wv[kk], acc[b], 0, 0, 0);
-            if (DUAL) {
-                const float* ur = &lu[buf][(16 * b + c) * kVLd + 8 * j];
-                const float4 u0 = *reinterpret_cast<const float4*>(ur), u1 = *reinterpret_cast<const float4*>(ur + 4);
-                const float uv[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-                for (int kk = 0; kk < 8; kk++)
-                    accu[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[kk], uv[kk], accu[b], 0, 0, 0);
-            }
         }
         if (s + 1 < S) lstore(buf ^ 1);
         __syncthreads();
     }
     // lane (c, j): acc[b][i] = C[row 16 wave + 4 j + i][col 16 b + c]
-    float v[4][4];
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[b][i] = acc[b][i];
-    if (g.ks > 1) {  // raw sums of this K slice
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int col = n0 + 16 * b + c;
-            if (col >= N) continue;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int row = m0 + 16 * wave + 4 * j + i;
-                if (row < g.M) g.part[((size_t)z * g.M + row) * N + col] = v[b][i];
-            }
-        }
-        return;
-    }
-    if ((EPI == VE_PLAIN || EPI == VE_QKV) && sg.bias)
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const float bb = bf2f(gld(sg.bias + min(ln0 + 16 * b + c, sg.n - 1)));
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[b][i] += bb;
-        }
-    if (EPI == VE_QKV && sg.rope)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) vrope(v[b][i], v[b + 2][i], 16 * b + c, m0 + 16 * wave + 4 * j + i, g.log2_theta);
 #pragma unroll
     for (int b = 0; b < 4; b++) {
         const int col = n0 + 16 * b + c;
-        if (col >= N) continue;
+        if (col >= g.n) continue;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int row = m0 + 16 * wave + 4 * j + i;
             if (row >= g.M) continue;
-            float o = v[b][i];
-            if (EPI == VE_RES) o = g.res[(size_t)row * g.ldres + col] + o;
-            if (EPI == VE_SWIGLU) {
-                const float sgm = 1.0f / (1.0f + expf(-o));
-                o = (o * sgm) * accu[b][i];
-            }
-            if (EPI == VE_WIN) o = o * g.win[col];
-            g.y[(size_t)row * g.ldy + col] = o;
+            if (g.ks > 1)  // raw sums of this K slice
+                g.part[((size_t)z * g.M + row) * g.n + col] = acc[b][i];
+            else
+                g.y[(size_t)row * g.n + col] = acc[b][i] * g.win[col];
         }
     }
 }
 
-// Split-K reduce + epilogue: thread = (row, 64-column tile, d < 32) owns the
-// columns d and d + 32 of the tile (a rotary pair); the ks partials are summed
-// in slice order.
-template <int EPI>
-__global__ __launch_bounds__(256) void vreduce_kernel(VGemm g) {
-    const int N = vtotal_n(g), tiles = (N + 63) / 64;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (int64_t)g.M * tiles * 32) return;
-    const int row = (int)(idx / (tiles * 32)), rem = (int)(idx % (tiles * 32)), tile = rem / 32, d = rem % 32;
-    int sstart;
-    const VSeg& sg = g.seg[vseg_of(g, tile * 64, sstart)];
-    float v[2];
-    bool ok[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int col = tile * 64 + d + 32 * h;
-        ok[h] = col < N;
-        float sum = 0.0f;
-        for (int z = 0; z < g.ks; z++) sum += ok[h] ? g.part[((size_t)z * g.M + row) * N + col] : 0.0f;
-        if ((EPI == VE_PLAIN || EPI == VE_QKV) && sg.bias && ok[h]) sum += bf2f(sg.bias[col - sstart]);
-        v[h] = sum;
-    }
-    if (EPI == VE_QKV && sg.rope) vrope(v[0], v[1], d, row, g.log2_theta);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        if (!ok[h]) continue;
-        const int col = tile * 64 + d + 32 * h;
-        float o = v[h];
-        if (EPI == VE_RES) o = g.res[(size_t)row * g.ldres + col] + o;
-        if (EPI == VE_WIN) o = o * g.win[col];
-        g.y[(size_t)row * g.ldy + col] = o;
-    }
-}
-
-// fast::rms_norm of f32 rows with a bf16 weight: w * (x * rsqrt(mean(x^2) + eps)); one wave per row.
-// Rows of K <= 1024, a multiple of 4: the row is read once, as up to four 16-byte chunks per lane held
-// in registers, so its loads are all in flight together.
-__global__ __launch_bounds__(256) void vrms4_kernel(const float* x, int M, int K, const uint16_t* w, float eps,
-                                                    float* out) {
-    const int row = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    if (row >= M) return;
-    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * K);
-    const int n4 = K / 4;
-    float4 v[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int c = lane + kWave * j;
-        v[j] = c < n4 ? xr[c] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-    float ss = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 4; j++) ss += (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w);
-    ss = team_sum<kWave>(ss);
-    const float inv = 1.0f / sqrtf(ss / (float)K + eps);
-    float4* o = reinterpret_cast<float4*>(out + (size_t)row * K);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int c = lane + kWave * j;
-        if (c < n4)
-            o[c] = make_float4(bf2f(gld(w + 4 * c)) * (v[j].x * inv), bf2f(gld(w + 4 * c + 1)) * (v[j].y * inv),
-                               bf2f(gld(w + 4 * c + 2)) * (v[j].z * inv), bf2f(gld(w + 4 * c + 3)) * (v[j].w * inv));
-    }
-}
-
-// Any K: two passes over the row, 4-byte accesses.
-__global__ __launch_bounds__(256) void vrms_kernel(const float* x, int M, int K, const uint16_t* w, float eps,
-                                                   float* out) {
-    const int row = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    if (row >= M) return;
-    const float* xr = x + (size_t)row * K;
-    float ss = 0.0f;
-    for (int i = lane; i < K; i += kWave) ss += xr[i] * xr[i];
-    ss = team_sum<kWave>(ss);
-    const float inv = 1.0f / sqrtf(ss / (float)K + eps);
-    for (int i = lane; i < K; i += kWave) out[(size_t)row * K + i] = bf2f(gld(w + i)) * (xr[i] * inv);
-}
-
-// Sliding-window attention (mask of src/ming_model.zig:618-636: key j is
-// visible to query i when i - window < j <= i, window <= 64), with the
-// window's K and V rows of one kv head staged in LDS once for the q heads that
-// share them: one workgroup per (row i, kv head), wave w = q head kh * grp + w
-// (grp <= 16): lane j scores key j0 + j, then lane = dim for P.V.  K rows are
-// padded to 68 floats so the lanes' 16-byte reads of 64 different rows spread
-// over the banks.
-constexpr int kVKs = 68;
-__global__ __launch_bounds__(1024) void vattn_gqa_kernel(const float* qkv, int M, int ldq, int H, int heads, int kvh,
-                                                         int window, float scale, float* att) {
-    __shared__ __align__(16) float ks[64 * kVKs];
-    __shared__ __align__(16) float vs[64 * 64];
-    const int i = blockIdx.x / kvh, kh = blockIdx.x % kvh, grp = heads / kvh;
-    const int j0 = max(0, i - window + 1), n = i - j0 + 1;
-    for (int f = threadIdx.x; f < 64 * 16; f += blockDim.x) {
-        const int r = f / 16, c4 = f % 16;
-        const float* base = qkv + (size_t)min(j0 + r, i) * ldq + H + kh * 64 + 4 * c4;
-        *reinterpret_cast<float4*>(ks + r * kVKs + 4 * c4) = *reinterpret_cast<const float4*>(base);
-        *reinterpret_cast<float4*>(vs + r * 64 + 4 * c4) = *reinterpret_cast<const float4*>(base + kvh * 64);
-    }
-    __syncthreads();
-    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave, h = kh * grp + w;
-    const float* q = qkv + (size_t)i * ldq + h * 64;
-    const float* kr = ks + lane * kVKs;
-    float p[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int d = 0; d < 64; d += 4) {
-        const float4 qa = *reinterpret_cast<const float4*>(q + d), ka = *reinterpret_cast<const float4*>(kr + d);
-        p[0] = fmaf(qa.x, ka.x, p[0]);
-        p[1] = fmaf(qa.y, ka.y, p[1]);
-        p[2] = fmaf(qa.z, ka.z, p[2]);
-        p[3] = fmaf(qa.w, ka.w, p[3]);
-    }
-    const float s = lane < n ? ((p[0] + p[1]) + (p[2] + p[3])) * scale : -INFINITY;
-    const float m = team_max<kWave>(s);
-    const float e = lane < n ? expf(s - m) : 0.0f;
-    const float l = team_sum<kWave>(e);
-    float o = 0.0f;
-#pragma unroll
-    for (int jj = 0; jj < 64; jj++) {
-        const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), jj));
-        o = fmaf(pj, vs[jj * 64 + lane], o);
-    }
-    att[(size_t)i * H + h * 64 + lane] = o / l;
-}
-
-// Decoder._linear_upsample_1d (align_corners=False, f32) of the fc1 rows,
-// which the graph materialises in bf16 first: y [T][C] f32 accumulators of
-// fc1 -> x [T * scale][C].  The fc1 row is bf16(acc + bias) for bf16
-// weights (addmm, one rounding) and bf16(bf16(acc) + bias) for 4-bit ones
-// (quantized_matmul, then the bias add).
-__device__ __forceinline__ float fc1_row(const float* y, const uint16_t* bias, int q4, int r, int C, int c) {
-    const float a = y[(size_t)r * C + c], b = bias ? bf2f(bias[c]) : 0.0f;
-    return q4 ? rb(rb(a) + b) : rb(a + b);
-}
-
-__global__ __launch_bounds__(256) void vup_kernel(const float* y, const uint16_t* bias, int q4, int T, int C, int scale,
-                                                  float* x) {
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (int64_t)T * scale * C) return;
-    const int i = (int)(idx / C), c = (int)(idx % C);
-    const float pos = ((float)i + 0.5f) / (float)scale - 0.5f;
-    const int left = (int)floorf(pos);
-    const float wr = pos - (float)left, wl = 1.0f - wr;
-    const int l = min(max(left, 0), T - 1), r = min(max(left + 1, 0), T - 1);
-    x[idx] = fc1_row(y, bias, q4, l, C, c) * wl + fc1_row(y, bias, q4, r, C, c) * wr;
+// The ks partials summed in slice order, then the window.
+__global__ __launch_bounds__(256) void vbasis_reduce_kernel(VBasis g) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n = (int64_t)g.M * g.n;
+    if (i >= n) return;
+    float sum = 0.0f;
+    for (int z = 0; z < g.ks; z++) sum += g.part[z * n + i];
+    g.y[i] = sum * g.win[i % g.n];
 }
 
 // ISTFT spectrum: p [F][n_fft + 2] (log-magnitudes | phases) -> the GEMM's
@@ -432,80 +241,37 @@ __global__ __launch_bounds__(256) void vwiden_kernel(const uint16_t* x, int64_t 
     if (i < n) y[i] = bf2f(x[i]);
 }
 
-template <int WF>
-hipError_t vgemm_wf(hipStream_t st, const VGemm& g, int epi, int N) {
-    const dim3 grid((N + kVBN - 1) / kVBN, (g.M + kVBM - 1) / kVBM, g.ks);
-    switch (epi) {
-        case VE_PLAIN: hipLaunchKernelGGL((vgemm_kernel<WF, VE_PLAIN>), grid, dim3(kVT), 0, st, g); break;
-        case VE_QKV: hipLaunchKernelGGL((vgemm_kernel<WF, VE_QKV>), grid, dim3(kVT), 0, st, g); break;
-        case VE_RES: hipLaunchKernelGGL((vgemm_kernel<WF, VE_RES>), grid, dim3(kVT), 0, st, g); break;
-        case VE_SWIGLU: hipLaunchKernelGGL((vgemm_kernel<WF, VE_SWIGLU>), grid, dim3(kVT), 0, st, g); break;
-        case VE_WIN: hipLaunchKernelGGL((vgemm_kernel<WF, VE_WIN>), grid, dim3(kVT), 0, st, g); break;
-        default: return hipErrorInvalidValue;
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || g.ks == 1) return e;
-    const int64_t items = (int64_t)g.M * ((N + 63) / 64) * 32;
-    const dim3 rg((unsigned)((items + 255) / 256));
-    switch (epi) {
-        case VE_PLAIN: hipLaunchKernelGGL((vreduce_kernel<VE_PLAIN>), rg, dim3(256), 0, st, g); break;
-        case VE_QKV: hipLaunchKernelGGL((vreduce_kernel<VE_QKV>), rg, dim3(256), 0, st, g); break;
-        case VE_RES: hipLaunchKernelGGL((vreduce_kernel<VE_RES>), rg, dim3(256), 0, st, g); break;
-        case VE_WIN: hipLaunchKernelGGL((vreduce_kernel<VE_WIN>), rg, dim3(256), 0, st, g); break;
-        default: return hipErrorInvalidValue;  // SwiGLU has no split form
-    }
-    return hipGetLastError();
-}
-
 }  // namespace
 
-// Host checks of a VGemm: segments start at multiples of 64, each K slice is
-// whole stages of 32 (and whole groups of 64 for affine weights), split K
-// has a partial buffer and no SwiGLU.
-static int vgemm_total_n(const VGemm& g) {
-    int n = 0;
-    for (int i = 0; i < g.nseg; i++) n += g.seg[i].n;
-    return n;
+bool vfft_plan(int n_fft, VFftPlan& p) {
+    p = VFftPlan{};
+    p.h = n_fft / 2;
+    if (n_fft % 2 || p.h < 2 || p.h > kFftMaxHalf) return false;
+    int r = p.h;
+    // fewest passes: 7s, 6s, 5s, then what is left of 4s, 3s and 2s
+    for (int f : {7, 6, 5, 4, 3, 2})
+        while (r % f == 0) {
+            if (p.passes == kFftMaxPasses) return false;
+            p.radix[p.passes++] = f;
+            r /= f;
+        }
+    return r == 1;
 }
 
-hipError_t launch_vgemm(hipStream_t st, const VGemm& g, int wf, int epi) {
-    if (g.nseg < 1 || g.nseg > 3 || g.ks < 1 || g.K % (kVBK * g.ks) || g.lda % 4 || g.M < 1) return hipErrorInvalidValue;
-    if (wf == VW_Q4 && (g.K / g.ks) % 64) return hipErrorInvalidValue;
-    for (int i = 0; i + 1 < g.nseg; i++)
-        if (g.seg[i].n % 64) return hipErrorInvalidValue;
-    if (g.ks > 1 && (!g.part || epi == VE_SWIGLU)) return hipErrorInvalidValue;
-    const int N = vgemm_total_n(g);
-    if (N < 1) return hipErrorInvalidValue;
-    if (wf == VW_BF16) return vgemm_wf<VW_BF16>(st, g, epi, N);
-    if (wf == VW_Q4) return vgemm_wf<VW_Q4>(st, g, epi, N);
-    if (wf == VW_F32) return vgemm_wf<VW_F32>(st, g, epi, N);
-    return hipErrorInvalidValue;
-}
-
-hipError_t launch_vrms(hipStream_t st, const float* x, int M, int K, const uint16_t* w, float eps, float* out) {
-    const bool v4 = K % 4 == 0 && K <= 4 * 4 * kWave && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-                    reinterpret_cast<uintptr_t>(out) % 16 == 0;
-    if (v4)
-        hipLaunchKernelGGL(vrms4_kernel, dim3((M + 3) / 4), dim3(256), 0, st, x, M, K, w, eps, out);
-    else
-        hipLaunchKernelGGL(vrms_kernel, dim3((M + 3) / 4), dim3(256), 0, st, x, M, K, w, eps, out);
+hipError_t launch_virfft(hipStream_t st, const VFftPlan& pl, const float* p, int F, const float* tw, const float* win,
+                         float* frames) {
+    if (pl.h < 2 || pl.h > kFftMaxHalf || F < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(virfft_kernel, dim3(F), dim3(256), 2 * sizeof(float2) * pl.h, st, pl, p,
+                       reinterpret_cast<const float2*>(tw), win, frames);
     return hipGetLastError();
 }
 
-hipError_t launch_vattn(hipStream_t st, const float* qkv, int M, int ldq, int H, int heads, int kvh, int window,
-                        float scale, float* att) {
-    if (window < 1 || window > 64 || kvh < 1 || heads % kvh) return hipErrorInvalidValue;
-    const int grp = heads / kvh;
-    if (grp > 16) return hipErrorInvalidValue;  // rejected at model creation
-    hipLaunchKernelGGL(vattn_gqa_kernel, dim3(M * kvh), dim3(64 * grp), 0, st, qkv, M, ldq, H, heads, kvh, window,
-                       scale, att);
-    return hipGetLastError();
-}
-
-hipError_t launch_vup(hipStream_t st, const float* y, const uint16_t* bias, int q4, int T, int C, int scale,
-                      float* x) {
-    const int64_t n = (int64_t)T * scale * C;
-    hipLaunchKernelGGL(vup_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, y, bias, q4, T, C, scale, x);
+hipError_t launch_vbasis(hipStream_t st, const VBasis& g) {
+    if (g.ks < 1 || g.K % (kVBK * g.ks) || g.M < 1 || g.n < 1 || (g.ks > 1 && !g.part)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(vbasis_kernel, dim3((g.n + kVBN - 1) / kVBN, (g.M + kVBM - 1) / kVBM, g.ks), dim3(kVT), 0, st, g);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || g.ks == 1) return e;
+    hipLaunchKernelGGL(vbasis_reduce_kernel, dim3((unsigned)(((int64_t)g.M * g.n + 255) / 256)), dim3(256), 0, st, g);
     return hipGetLastError();
 }
 
