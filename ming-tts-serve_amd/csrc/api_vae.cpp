@@ -36,6 +36,8 @@ constexpr int kMaxSlices = 8;
 
 int vae_err(ming_ctx* ctx, int st, const std::string& m) { return set_err(ctx, st, "vae: " + m); }
 
+int is_q4(const ming_linear& l) { return linear_dev(l).kind == 1; }
+
 // The weight of a linear as a GEMM segment; wf receives its format.
 VSeg seg_of(const ming_linear& l, const void* bias, int rope, int& wf) {
     const LinearDev d = linear_dev(l);
@@ -53,11 +55,10 @@ VSeg seg_of(const ming_linear& l, const void* bias, int rope, int& wf) {
 
 // K slices of a residual projection: the row kernel after it adds the partials
 // either way, so a split costs only their traffic.  Few rows: slices of at most
-// eight waves' chunks (K = 4864: 5), so that no wave loops and N / 16 = 56
-// workgroups become 280.  Many rows: enough 64 x 64 tiles to cover the 256 CUs.
+// ten waves' chunks of 128 (K = 4864: 4), so that no wave loops and N / 16 = 56
+// workgroups become 224.  Many rows: enough 64 x 64 tiles to cover the 256 CUs.
 int split_k(int M, int N, int K) {
-    const int blocks = M <= kV3SmallRows ? (K / 32 + 31) / 32 : 1;
-    if (M <= kV3SmallRows) return std::min(kMaxSlices, K > 1024 ? blocks : 1);
+    if (M <= kV3SmallRows) return std::min(kMaxSlices, (K + 1279) / 1280);
     if (K <= 1024) return 1;  // 32 x 64 tiles
     const int tiles = ((N + 63) / 64) * ((M + 63) / 64);
     int ks = 1;
@@ -161,12 +162,13 @@ int ming_vae_model_create(ming_ctx* ctx, const ming_vae_cfg* cfg, const ming_vae
         if (e == hipSuccess) e = hipMemcpy(m->basis.p, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = m->spec.ensure(F * m->ldspec * sizeof(float));
     }
+    const size_t Fp = (F + 15) / 16 * 16;  // rows of a plane
     const size_t part_cols = m->ldspec ? std::max((size_t)H, (size_t)N) : (size_t)H;
     const std::pair<DevBuf*, size_t> bufs[] = {  // bytes
         {&m->lat, (size_t)max_latents * cfg->latent * 2}, {&m->xs, (cfg->n_layers + 1) * F * H * 4},
-        {&m->h, 3 * F * H * 2},                           {&m->qkv, F * nq * 4},
-        {&m->att, 3 * F * H * 2},                         {&m->x1, F * H * 4},
-        {&m->hh, 3 * F * I * 2},                          {&m->p, F * P * 4},
+        {&m->h, 3 * Fp * H * 2},                          {&m->qkv, F * nq * 4},
+        {&m->att, 3 * Fp * H * 2},                        {&m->x1, F * H * 4},
+        {&m->hh, 3 * Fp * I * 2},                         {&m->p, F * P * 4},
         {&m->frames, F * N * 4},                          {&m->part, kMaxSlices * F * part_cols * 4},
         {&m->rope, F * 64 * 4}};
     for (const auto& b : bufs)
@@ -199,6 +201,7 @@ int ming_vae_decode(ming_ctx* ctx, ming_vae_model* m, int32_t T, const void* lat
     const ming_vae_cfg& c = m->cfg;
     const int H = c.hidden, kvd = c.kv_heads * c.head_dim, I = c.inter, nq = H + 2 * kvd, P = c.n_fft + 2;
     const int F = T * c.patch;
+    const size_t Fp = (size_t)(F + 15) / 16 * 16;  // rows of a plane
     hipStream_t st = ctx->stream;
     float *xs = static_cast<float*>(m->xs.p), *qkv = static_cast<float*>(m->qkv.p), *x1 = static_cast<float*>(m->x1.p);
     float* part = static_cast<float*>(m->part.p);
@@ -209,7 +212,7 @@ int ming_vae_decode(ming_ctx* ctx, ming_vae_model* m, int32_t T, const void* lat
     auto gemm = [&](const uint16_t* a, int M, int K, float* y, int ldy) {
         V3Gemm g{};
         g.a = a;
-        g.aps = (size_t)M * K;
+        g.aps = Fp * K;
         g.np = 3;
         g.M = M;
         g.K = K;
@@ -232,7 +235,7 @@ int ming_vae_decode(ming_ctx* ctx, ming_vae_model* m, int32_t T, const void* lat
         if (e == hipSuccess) e = launch_v3gemm(st, g, wf, VE_PLAIN);
     }
     // x = (res + the partials) or the upsampled rows, and h = rms_norm(x) for the next linear
-    auto row = [&](const float* res, float* x, int ks, const void* norm, bool up) {
+    auto row = [&](const float* res, float* x, int ks, const void* norm, bool up, const ming_linear& next) {
         VRowArgs a{};
         a.part = part;
         a.ks = ks;
@@ -243,14 +246,15 @@ int ming_vae_decode(ming_ctx* ctx, ming_vae_model* m, int32_t T, const void* lat
         a.w = static_cast<const uint16_t*>(norm);
         a.eps = c.eps;
         a.h = h;
-        a.hps = (size_t)F * H;
+        a.hps = Fp * H;
+        a.hpair = is_q4(next);
         a.bias = m->fc1_bias;
         a.q4 = wf == VW_Q4;
         a.T = T;
         a.scale = c.patch;
         return launch_vrow(st, a, up);
     };
-    if (e == hipSuccess) e = row(nullptr, xs, 0, m->layers[0].ln1, true);
+    if (e == hipSuccess) e = row(nullptr, xs, 0, m->layers[0].ln1, true, m->layers[0].wq);
     const float scale = 1.0f / std::sqrt((float)c.head_dim);
     const int ks_o = split_k(F, H, H), ks_d = split_k(F, H, I);
     for (int l = 0; l < c.n_layers && e == hipSuccess; l++) {
@@ -266,21 +270,22 @@ int ming_vae_decode(ming_ctx* ctx, ming_vae_model* m, int32_t T, const void* lat
             e = launch_v3gemm(st, g, wf, VE_QKV);
         }
         if (e == hipSuccess)
-            e = launch_vattn(st, qkv, F, nq, H, c.heads, c.kv_heads, c.window, scale, att, (size_t)F * H);
+            e = launch_vattn(st, qkv, F, nq, H, c.heads, c.kv_heads, c.window, scale, att, Fp * H, is_q4(L.wo));
         if (e == hipSuccess) {
             V3Gemm g = gemm(att, F, H, part, H);
             g.seg[0] = seg_of(L.wo, nullptr, 0, wf);
             g.ks = ks_o;
             e = launch_v3gemm(st, g, wf, VE_RES);
         }
-        if (e == hipSuccess) e = row(x, x1, ks_o, L.ln2, false);
+        if (e == hipSuccess) e = row(x, x1, ks_o, L.ln2, false, L.wg);
         if (e == hipSuccess) {
             V3Gemm g = gemm(h, F, H, nullptr, 0);
             g.seg[0] = seg_of(L.wg, nullptr, 0, wf);
             g.up = seg_of(L.wu, nullptr, 0, wf);
             g.yp = hh;
-            g.yps = (size_t)F * I;
+            g.yps = Fp * I;
             g.ldyp = I;
+            g.ypair = is_q4(L.wd);
             e = launch_v3gemm(st, g, wf, VE_SWIGLU);
         }
         if (e == hipSuccess) {
@@ -289,7 +294,9 @@ int ming_vae_decode(ming_ctx* ctx, ming_vae_model* m, int32_t T, const void* lat
             g.ks = ks_d;
             e = launch_v3gemm(st, g, wf, VE_RES);
         }
-        if (e == hipSuccess) e = row(x1, xo, ks_d, l + 1 < c.n_layers ? m->layers[l + 1].ln1 : m->norm, false);
+        const bool last = l + 1 == c.n_layers;
+        if (e == hipSuccess)
+            e = row(x1, xo, ks_d, last ? m->norm : m->layers[l + 1].ln1, false, last ? m->head : m->layers[l + 1].wq);
     }
     float *p = static_cast<float*>(m->p.p), *frames = static_cast<float*>(m->frames.p);
     if (e == hipSuccess) {

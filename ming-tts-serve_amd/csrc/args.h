@@ -143,7 +143,9 @@ struct VSeg {
 // columns one after another (N = sum of seg[i].n).
 constexpr int kV3SmallRows = 64;  // rows up to which the unstaged kernel runs
 struct V3Gemm {
-    const uint16_t* a;      // bf16 planes [np][M][K] whose sum is A (np = 3, or 1 for a bf16 input)
+    // np = 3: bf16 planes whose sum is A, in operand order (vae_gemm.hip), rows padded to 16;
+    // np = 1: bf16 [M][K]
+    const uint16_t* a;
     size_t aps;             // values between planes
     int np, M, K;
     VSeg seg[3];
@@ -151,9 +153,9 @@ struct V3Gemm {
     VSeg up;                // VE_SWIGLU
     float* y;
     int ldy;
-    uint16_t* yp;           // VE_SWIGLU: bf16 planes [3][M][ldyp]
+    uint16_t* yp;           // VE_SWIGLU: the output's planes (ldyp columns)
     size_t yps;
-    int ldyp;
+    int ldyp, ypair;        // ypair: the planes' consumer has 4-bit weights
     const float* rope_cs;   // VE_QKV: f32 [rows][32][2] (cos, sin)
     int ks;                 // VE_RES: K slices
 };
@@ -169,8 +171,9 @@ struct VRowArgs {
     int M, N;
     const uint16_t* w;      // bf16 [N]
     float eps;
-    uint16_t* h;            // bf16 [3][M][N]
+    uint16_t* h;            // planes of N columns
     size_t hps;
+    int hpair;              // the planes' consumer has 4-bit weights
     const uint16_t* bias;   // upsample: fc1's bias (bf16 [N] or null), format, latents, factor
     int q4, T, scale;
 };

@@ -141,7 +141,7 @@ bool lm_model_view(const ming_lm_model* m, LmView& v);
 hipError_t launch_v3gemm(hipStream_t st, const V3Gemm& g, int wf, int epi);
 hipError_t launch_vrow(hipStream_t st, const VRowArgs& a, bool upsample);
 hipError_t launch_vattn(hipStream_t st, const float* qkv, int M, int ldq, int H, int heads, int kvh, int window,
-                        float scale, uint16_t* att, size_t aps);
+                        float scale, uint16_t* att, size_t aps, int pair);
 // The passes for an n_fft-point inverse real FFT; false when n_fft / 2 has a
 // prime factor above 7 or does not fit the kernel's LDS.
 bool vfft_plan(int n_fft, VFftPlan& p);

@@ -8,12 +8,20 @@
 // a fifth of their cost (dense bf16 against f32: 1213 against 154 TFLOP/s for
 // a library product on this card).  The high plane's sum and the two low
 // planes' sum are kept apart and added once, so the low planes' roundings fall
-// below the last bit.  4-bit weights enter as the exact integers q - 8; each
-// group of 64 is folded in f32 as s * sum (q - 8) x + (b + 8 s) * sum x, the
-// group sums of x coming from the same MFMAs against a column of ones.
+// below the last bit.  4-bit weights enter as the exact values 16 + q (a nibble
+// OR-ed into bits 3..6 of bf16(16): two instructions a pair, where converting
+// q - 8 took five); each group of 64 is folded in f32 as s * sum (16 + q) x +
+// (b - 16 s) * sum x, the group sums of x coming from the same MFMAs against a
+// column of ones, and within a group the low planes are summed first, so only
+// the high plane's two MFMAs round at the sum's own size.
 //
-// Activations therefore travel between the kernels as planes: bf16 [3][M][K]
-// (fc1's bf16 input is one plane), written by the kernel that produces them.
+// Activations therefore travel between the kernels as planes, written by the
+// kernel that produces them in the MFMA A operand's order: bf16 [3][M / 16]
+// [K / 32][lane][8], lane = 16 (k % 32 / 8) + m % 16 (plane_at), so that a
+// wave's operand is one contiguous KiB.  (Row-major planes made each operand
+// load 16 half-used cache lines.)  For 4-bit weights the 8 values lie in the
+// unpacked word's pair order (0, 4), (1, 5), (2, 6), (3, 7).  fc1's bf16 input
+// stays row-major in natural order, one plane.
 //
 // Two kernels.  vsmall_kernel (few rows): no LDS staging, the waves of a
 // workgroup split K and stream their operands straight into registers, which
@@ -33,17 +41,6 @@ __device__ __forceinline__ int v3_total_n(const V3Gemm& g) {
     return g.seg[0].n + (g.nseg > 1 ? g.seg[1].n : 0) + (g.nseg > 2 ? g.seg[2].n : 0);
 }
 
-// The segment holding output column c (segments start at multiples of 64) and its first column.
-__device__ __forceinline__ int v3_seg_of(const V3Gemm& g, int c, int& start) {
-    start = 0;
-    int i = 0;
-    while (i + 1 < g.nseg && c >= start + g.seg[i].n) {
-        start += g.seg[i].n;
-        i++;
-    }
-    return i;
-}
-
 // x = p[0] + p[1] + p[2] exactly, each a bf16 (as f32 bits with a zero low half): truncations
 // leave 16, then 8 significant bits, so both differences are exact.  An infinity is its own
 // first plane (the others 0) and a NaN stays one.
@@ -57,13 +54,32 @@ __device__ __forceinline__ void split3(float x, uint32_t (&p)[3]) {
 // The high halves of two words as a bf16 pair (lo in the low half).
 __device__ __forceinline__ uint32_t hi_pair(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
 
-// 8 nibbles of a packed word as the bf16 values q - 8 in natural order (exact integers).
-__device__ __forceinline__ uint4 unpack_q8(uint32_t w) {
-    const int32_t x = (int32_t)(w ^ 0x88888888u);  // q - 8 as a signed 4-bit field
-    uint32_t f[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) f[i] = __float_as_uint((float)((int32_t)((uint32_t)x << (28 - 4 * i)) >> 28));
-    return make_uint4(hi_pair(f[0], f[1]), hi_pair(f[2], f[3]), hi_pair(f[4], f[5]), hi_pair(f[6], f[7]));
+// 8 nibbles of a packed word as the bf16 values 16 + q (exact) in pair order: nibble i and
+// i + 4 are one pair.
+__device__ __forceinline__ uint4 unpack_q16(uint32_t w, uint32_t mask, uint32_t magic) {
+    return make_uint4(((w << 3) & mask) | magic, ((w >> 1) & mask) | magic, ((w >> 5) & mask) | magic,
+                      ((w >> 9) & mask) | magic);
+}
+constexpr uint32_t kQ16Mask = 0x00780078u, kQ16Magic = 0x41804180u;
+
+// A value the compiler must keep in a register: mask and magic then make one v_and_or_b32
+// (which takes no literal operands).
+__device__ __forceinline__ uint32_t in_reg(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// The operand of 8 natural-order values in pair order.
+__device__ __forceinline__ uint4 pair_order(uint4 e) {
+    return make_uint4(__builtin_amdgcn_perm(e.z, e.x, 0x05040100u), hi_pair(e.x, e.z),
+                      __builtin_amdgcn_perm(e.w, e.y, 0x05040100u), hi_pair(e.y, e.w));
+}
+
+// Place of value (row m, column k) in a plane of K columns; pair: the consumer's weights are 4-bit.
+__device__ __forceinline__ size_t plane_at(int m, int k, int K, int pair) {
+    const int e = k % 8;
+    return ((size_t)(m / 16) * (K / 32) + k / 32) * 512 + (16 * (k % 32 / 8) + m % 16) * 8 +
+           (pair ? 2 * (e % 4) + e / 4 : e);
 }
 
 __device__ __forceinline__ f32x4_t mma(uint4 a, uint4 b, f32x4_t c) {
@@ -72,9 +88,95 @@ __device__ __forceinline__ f32x4_t mma(uint4 a, uint4 b, f32x4_t c) {
 
 constexpr f32x4_t kZero4 = {0.0f, 0.0f, 0.0f, 0.0f};
 
+// What a workgroup needs of its arguments, read in one go (load_view): the argument block's
+// scalar loads are a chain of cold misses (0.3 - 0.7 us each) when a kernel picks its segment
+// by index and reads each field where it is used.
+template <int WF, int EPI>
+struct V3View {
+    const char *w, *wu;              // weights: the block's segment, up
+    const uint16_t *s, *b, *su, *bu;  // affine scales and biases
+    const uint16_t* bias;
+    float gs, gu;
+    int n, start, rope;  // the segment's columns, its first column, rotary
+    int M, K, ks, ldy, ldyp, ypair;
+    const uint16_t* a;
+    size_t aps, yps;
+    float* y;
+    uint16_t* yp;
+    const float* rope_cs;
+};
+
+#define MING_PIN(...) asm volatile("" : __VA_ARGS__)
+#define MING_S(x) "+s"(x)
+
+// The view of the segment that holds output column c0 (segments start at multiples of 64).
+template <int WF, int EPI>
+__device__ __forceinline__ V3View<WF, EPI> load_view(const V3Gemm& g, int c0) {
+    V3View<WF, EPI> v;
+    VSeg s0 = g.seg[0], s1 = EPI == VE_SWIGLU ? g.up : g.seg[1], s2 = g.seg[2];
+    v.M = g.M;
+    v.K = g.K;
+    v.ks = g.ks;
+    v.a = g.a;
+    v.aps = g.aps;
+    v.y = g.y;
+    v.ldy = g.ldy;
+    v.yp = g.yp;
+    v.yps = g.yps;
+    v.ldyp = g.ldyp;
+    v.ypair = g.ypair;
+    v.rope_cs = g.rope_cs;
+    // all that this kernel reads in registers here, before anything depends on any of it
+    if constexpr (EPI == VE_SWIGLU) {
+        if constexpr (WF == VW_Q4)
+            MING_PIN(MING_S(s0.w), MING_S(s0.gs), MING_S(s0.n), MING_S(v.M), MING_S(v.K), MING_S(v.a), MING_S(s0.s),
+                     MING_S(s0.b), MING_S(s1.w), MING_S(s1.gs), MING_S(v.yp), MING_S(v.ldyp), MING_S(v.ypair),
+                     MING_S(s1.s), MING_S(s1.b));
+        else
+            MING_PIN(MING_S(s0.w), MING_S(s0.gs), MING_S(s0.n), MING_S(v.M), MING_S(v.K), MING_S(v.a), MING_S(s1.w),
+                     MING_S(s1.gs), MING_S(v.yp), MING_S(v.ldyp), MING_S(v.ypair));
+        MING_PIN(MING_S(v.yps), MING_S(v.aps));
+    } else if constexpr (EPI == VE_QKV) {
+        MING_PIN(MING_S(s0.w), MING_S(s0.n), MING_S(s1.w), MING_S(s1.n), MING_S(s2.w), MING_S(s2.n), MING_S(v.M),
+                 MING_S(v.K), MING_S(v.a), MING_S(v.aps), MING_S(v.y), MING_S(v.ldy), MING_S(v.rope_cs));
+        if constexpr (WF == VW_Q4)
+            MING_PIN(MING_S(s0.s), MING_S(s0.b), MING_S(s1.s), MING_S(s1.b), MING_S(s2.s), MING_S(s2.b));
+        MING_PIN(MING_S(s0.gs), MING_S(s0.bias), MING_S(s0.rope), MING_S(s1.gs), MING_S(s1.bias), MING_S(s1.rope),
+                 MING_S(s2.gs), MING_S(s2.bias), MING_S(s2.rope));
+    } else {
+        MING_PIN(MING_S(s0.w), MING_S(s0.gs), MING_S(s0.n), MING_S(v.M), MING_S(v.K), MING_S(v.a), MING_S(v.aps),
+                 MING_S(v.y), MING_S(v.ldy), MING_S(v.ks), MING_S(s0.bias), MING_S(s0.s), MING_S(s0.b));
+    }
+    v.start = 0;
+    if (EPI == VE_QKV) {
+        const int e0 = s0.n, e1 = s0.n + s1.n;
+        if (c0 >= e1) {
+            s0 = s2;
+            v.start = e1;
+        } else if (c0 >= e0) {
+            s0 = s1;
+            v.start = e0;
+        }
+        v.rope = s0.rope;
+    }
+    v.w = static_cast<const char*>(s0.w);
+    v.gs = s0.gs;
+    v.n = s0.n;
+    v.bias = s0.bias;
+    v.s = s0.s;
+    v.b = s0.b;
+    if (EPI == VE_SWIGLU) {
+        v.wu = static_cast<const char*>(s1.w);
+        v.su = s1.s;
+        v.bu = s1.b;
+        v.gu = s1.gs;
+    }
+    return v;
+}
+
 // MLX fast::rope of the pair (d, d + 32) of a 64-column head from the table's (cos, sin).
-__device__ __forceinline__ void v3_rope(const V3Gemm& g, int row, int d, float& x1, float& x2) {
-    const float2 cs = *reinterpret_cast<const float2*>(g.rope_cs + ((size_t)row * 32 + d) * 2);
+__device__ __forceinline__ void v3_rope(const float* rope_cs, int row, int d, float& x1, float& x2) {
+    const float2 cs = *reinterpret_cast<const float2*>(rope_cs + ((size_t)row * 32 + d) * 2);
     const float a = x1, b = x2;
     x1 = a * cs.x - b * cs.y;
     x2 = a * cs.y + b * cs.x;
@@ -82,41 +184,36 @@ __device__ __forceinline__ void v3_rope(const V3Gemm& g, int row, int d, float& 
 
 __device__ __forceinline__ float v3_swiglu(float g, float u) { return (g * (1.0f / (1.0f + expf(-g)))) * u; }
 
-// One value of the swiglu product into the three planes of the next linear's input.
-__device__ __forceinline__ void store_planes(const V3Gemm& g, int row, int col, float o) {
-    uint32_t p[3];
-    split3(o, p);
-    uint16_t* y = g.yp + (size_t)row * g.ldyp + col;
-#pragma unroll
-    for (int k = 0; k < 3; k++) gst(y + k * g.yps, (uint16_t)(p[k] >> 16));
-}
-
-// The epilogue of one row: v[t] are the sums of this lane's columns col[t] (of segment sg that
-// starts at sstart); QKV holds rotary pairs in (t, t + NT / 2), SWIGLU gate and up likewise.
-template <int EPI, int NT>
-__device__ __forceinline__ void v3_epi(const V3Gemm& g, const VSeg& sg, int sstart, int row, const int (&col)[NT],
-                                       float (&v)[NT], int z) {
+// The epilogue of one row: x[t] are the sums of this lane's columns col[t]; QKV holds rotary
+// pairs in (t, t + NT / 2), SWIGLU gate and up likewise.
+template <int WF, int EPI, int NT>
+__device__ __forceinline__ void v3_epi(const V3View<WF, EPI>& v, int row, const int (&col)[NT], float (&x)[NT], int z) {
     if constexpr (EPI == VE_SWIGLU) {
 #pragma unroll
-        for (int t = 0; t < NT / 2; t++)
-            store_planes(g, row, col[t], v3_swiglu(v[t] * sg.gs, v[t + NT / 2] * g.up.gs));
+        for (int t = 0; t < NT / 2; t++) {  // into the planes of the next linear's input
+            uint32_t p[3];
+            split3(v3_swiglu(x[t] * v.gs, x[t + NT / 2] * v.gu), p);
+            uint16_t* y = v.yp + plane_at(row, col[t], v.ldyp, v.ypair);
+#pragma unroll
+            for (int k = 0; k < 3; k++) gst(y + k * v.yps, (uint16_t)(p[k] >> 16));
+        }
     } else if constexpr (EPI == VE_RES) {  // this K slice's sums; the row kernel adds them to the residual
 #pragma unroll
         for (int t = 0; t < NT; t++)
-            if (col[t] < sg.n) gst(g.y + ((size_t)z * g.M + row) * g.ldy + col[t], v[t] * sg.gs);
+            if (col[t] < v.n) gst(v.y + ((size_t)z * v.M + row) * v.ldy + col[t], x[t] * v.gs);
     } else {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            v[t] *= sg.gs;
-            if (sg.bias) v[t] += bf2f(gld(sg.bias + min(col[t] - sstart, sg.n - 1)));
+            x[t] *= v.gs;
+            if (v.bias) x[t] += bf2f(gld(v.bias + min(col[t] - v.start, v.n - 1)));
         }
         if constexpr (EPI == VE_QKV)
-            if (sg.rope)
+            if (v.rope)
 #pragma unroll
-                for (int t = 0; t < NT / 2; t++) v3_rope(g, row, col[t] % 64, v[t], v[t + NT / 2]);
+                for (int t = 0; t < NT / 2; t++) v3_rope(v.rope_cs, row, col[t] % 64, x[t], x[t + NT / 2]);
 #pragma unroll
         for (int t = 0; t < NT; t++)
-            if (col[t] - sstart < sg.n) gst(g.y + (size_t)row * g.ldy + col[t], v[t]);
+            if (col[t] - v.start < v.n) gst(v.y + (size_t)row * v.ldy + col[t], x[t]);
     }
 }
 
@@ -124,55 +221,53 @@ __device__ __forceinline__ void v3_epi(const V3Gemm& g, const VSeg& sg, int ssta
 // Workgroup (column block x, row block of 16 MT rows y, K slice z); its waves split the
 // slice's units (32 k for bf16 weights, one group of 64 for affine ones) in chunks of CH
 // whose loads are all issued before the chunk's MFMAs, and their sums meet in LDS in wave
-// order.  Columns of a block: 16 (PLAIN, RES), 16 gate + 16 up (SWIGLU), or 16 and the 16
+// order.  Columns of a block: 16 (PLAIN, RES), 32 gate + 32 up (SWIGLU), or 16 and the 16
 // that are 32 further in the same head (QKV: rotary pairs meet in one lane).
 template <int WF>
 constexpr int kUnitK = WF == VW_Q4 ? 64 : 32;
 template <int WF>
 constexpr int kSmallCh = WF == VW_Q4 ? 2 : 4;
-constexpr int kSmallWaves = 8;
+template <int EPI>
+constexpr int kSmallNT = EPI == VE_SWIGLU ? 4 : (EPI == VE_QKV ? 2 : 1);
+// most waves of a workgroup: what their registers allow (one column tile: three a SIMD)
+template <int EPI>
+constexpr int kSmallWaves = kSmallNT<EPI> == 1 ? 10 : 8;
 
 template <int WF, int NP, int MT, int NT>
 struct V3Unit {
     uint4 a[kUnitK<WF> / 32][NP][MT];
     uint4 w[WF == VW_Q4 ? 1 : NT];
-    uint2 q[WF == VW_Q4 ? NT : 1];
+    uint32_t q[WF == VW_Q4 ? NT : 1][2];
     uint16_t s[NT], b[NT];
 };
 
 template <int WF, int EPI, int NP, int MT>
-__global__ __launch_bounds__(64 * kSmallWaves) void vsmall_kernel(V3Gemm g) {
-    constexpr int NT = EPI == VE_QKV || EPI == VE_SWIGLU ? 2 : 1;
+__global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g) {
+    constexpr int NT = kSmallNT<EPI>;
     constexpr int UK = kUnitK<WF>, UH = UK / 32, CH = kSmallCh<WF>;
     extern __shared__ float red[];  // [waves][MT * 4][NT][64]
     const int W = blockDim.x / kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave, c = lane % 16, j = lane / 16;
     const int m0 = blockIdx.y * 16 * MT, z = blockIdx.z;
+    const int c0 = EPI == VE_QKV ? (blockIdx.x / 2) * 64 + (blockIdx.x % 2) * 16 : blockIdx.x * (EPI == VE_SWIGLU ? 32 : 16);
     int col[NT];
 #pragma unroll
-    for (int t = 0; t < NT; t++)
-        col[t] = EPI == VE_QKV ? (blockIdx.x / 2) * 64 + (blockIdx.x % 2) * 16 + 32 * t + c : blockIdx.x * 16 + c;
-    int sstart;
-    const VSeg& sg = g.seg[v3_seg_of(g, EPI == VE_QKV ? (blockIdx.x / 2) * 64 : blockIdx.x * 16, sstart)];
-    const int U = g.K / UK, per = (U + g.ks - 1) / g.ks, u0 = z * per, u1 = min(U, u0 + per);
-    const uint16_t* ar[MT];
+    for (int t = 0; t < NT; t++) col[t] = c0 + (EPI == VE_QKV ? 32 * t : 16 * (t % 2)) + c;
+    const V3View<WF, EPI> v = load_view<WF, EPI>(g, c0);
+    const int U = v.K / UK, per = (U + v.ks - 1) / v.ks, u0 = z * per, u1 = min(U, u0 + per);
+    // 32-bit byte offsets per lane from uniform bases (operands: row tile; weights: row)
+    uint32_t ao[MT], wo[NT], so[NT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
-        ar[mt] = g.a + (size_t)min(m0 + 16 * mt + c, g.M - 1) * g.K + (WF == VW_Q4 ? 16 : 8) * j;
-    const char* wr[NT];
-    const uint16_t *sr[NT], *br[NT];
+        ao[mt] = NP == 1 ? (uint32_t)min(m0 + 16 * mt + c, v.M - 1) * v.K * 2u + 16u * j
+                         : (uint32_t)min(m0 / 16 + mt, (v.M - 1) / 16) * (v.K / 32) * 1024u + 16u * lane;
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        const VSeg& s = EPI == VE_SWIGLU && t == 1 ? g.up : sg;
-        const int n = min(col[t] - sstart, s.n - 1);
-        if (WF == VW_Q4) {
-            wr[t] = static_cast<const char*>(s.w) + (size_t)n * (g.K / 2) + 8 * j;
-            sr[t] = s.s + (size_t)n * (g.K / 64);
-            br[t] = s.b + (size_t)n * (g.K / 64);
-        } else {
-            wr[t] = static_cast<const char*>(s.w) + (size_t)n * g.K * 2 + 16 * j;
-        }
+        const uint32_t n = min(col[t] - v.start, v.n - 1);
+        wo[t] = WF == VW_Q4 ? n * (v.K / 2) + 4u * j : n * v.K * 2u + 16u * j;
+        so[t] = n * (v.K / 64) * 2u;
     }
+    auto at = [](const void* base, uint32_t off) { return static_cast<const char*>(base) + off; };
     f32x4_t hi[MT][NT], lo[MT][NT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
@@ -181,14 +276,16 @@ __global__ __launch_bounds__(64 * kSmallWaves) void vsmall_kernel(V3Gemm g) {
     auto load = [&](int u, V3Unit<WF, NP, MT, NT>& in) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
+            const bool up = EPI == VE_SWIGLU && t >= NT / 2;
+            const char* w = up ? v.wu : v.w;
             if (WF == VW_Q4) {
-                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-                const u32x2 v = *(const MING_GLOBAL u32x2*)(wr[t] + 32 * (size_t)u);
-                in.q[t] = make_uint2(v.x, v.y);
-                in.s[t] = gld(sr[t] + u);
-                in.b[t] = gld(br[t] + u);
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    in.q[t][h] = gld(reinterpret_cast<const uint32_t*>(at(w + 32 * (size_t)u + 16 * h, wo[t])));
+                in.s[t] = gld(reinterpret_cast<const uint16_t*>(at((up ? v.su : v.s) + u, so[t])));
+                in.b[t] = gld(reinterpret_cast<const uint16_t*>(at((up ? v.bu : v.b) + u, so[t])));
             } else {
-                in.w[t] = ldg4(wr[t] + 64 * (size_t)u);
+                in.w[t] = ldg4(at(w + 64 * (size_t)u, wo[t]));
             }
         }
 #pragma unroll
@@ -196,31 +293,39 @@ __global__ __launch_bounds__(64 * kSmallWaves) void vsmall_kernel(V3Gemm g) {
 #pragma unroll
             for (int p = 0; p < NP; p++)
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++) in.a[h][p][mt] = ldg4(ar[mt] + p * g.aps + (size_t)u * UK + 8 * h);
+                for (int mt = 0; mt < MT; mt++)
+                    in.a[h][p][mt] = ldg4(at(v.a + p * v.aps + ((size_t)u * UH + h) * (NP == 1 ? 32 : 512), ao[mt]));
     };
     const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+    const uint32_t mask = in_reg(kQ16Mask), magic = in_reg(kQ16Magic);
     auto work = [&](const V3Unit<WF, NP, MT, NT>& in) {
         if constexpr (WF == VW_Q4) {
-            f32x4_t xs[MT];  // group sums of x, in every column's place
+            // the group sums of x, in every column's place
+            f32x4_t xs[MT];
+            uint4 x[2][NP][MT];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int p = 0; p < NP; p++)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) x[h][p][mt] = NP == 1 ? pair_order(in.a[h][p][mt]) : in.a[h][p][mt];
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
-                f32x4_t h = mma(in.a[1][0][mt], ones, mma(in.a[0][0][mt], ones, kZero4)), l = kZero4;
+                xs[mt] = kZero4;
 #pragma unroll
-                for (int p = 1; p < NP; p++) l = mma(in.a[1][p][mt], ones, mma(in.a[0][p][mt], ones, l));
-                xs[mt] = h + l;
+                for (int p = NP - 1; p >= 0; p--) xs[mt] = mma(x[1][p][mt], ones, mma(x[0][p][mt], ones, xs[mt]));
             }
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                const uint4 b0 = unpack_q8(in.q[t].x), b1 = unpack_q8(in.q[t].y);
-                const float s = bf2f(in.s[t]), off = fmaf(8.0f, s, bf2f(in.b[t]));
+                const uint4 b0 = unpack_q16(in.q[t][0], mask, magic), b1 = unpack_q16(in.q[t][1], mask, magic);
+                const float s = bf2f(in.s[t]), off = fmaf(-16.0f, s, bf2f(in.b[t]));
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) {
-                    f32x4_t h = mma(in.a[1][0][mt], b1, mma(in.a[0][0][mt], b0, kZero4)), l = kZero4;
+                    f32x4_t h = kZero4;
 #pragma unroll
-                    for (int p = 1; p < NP; p++) l = mma(in.a[1][p][mt], b1, mma(in.a[0][p][mt], b0, l));
+                    for (int p = NP - 1; p >= 0; p--) h = mma(x[1][p][mt], b1, mma(x[0][p][mt], b0, h));
 #pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        hi[mt][t][r] = fmaf(s, h[r] + l[r], fmaf(off, xs[mt][r], hi[mt][t][r]));
+                    for (int r = 0; r < 4; r++) hi[mt][t][r] = fmaf(s, h[r], fmaf(off, xs[mt][r], hi[mt][t][r]));
                 }
             }
         } else {
@@ -235,7 +340,9 @@ __global__ __launch_bounds__(64 * kSmallWaves) void vsmall_kernel(V3Gemm g) {
                     }
         }
     };
-    for (int u = u0 + wave * CH; u < u1; u += W * CH) {
+    for (int ub = u0 + wave * CH; ub < u1; ub += W * CH) {
+        // a fresh scalar each time round: the loads keep their uniform base + lane offset form
+        const int u = __builtin_amdgcn_readfirstlane(ub);
         V3Unit<WF, NP, MT, NT> in[CH];
 #pragma unroll
         for (int k = 0; k < CH; k++)
@@ -254,30 +361,32 @@ __global__ __launch_bounds__(64 * kSmallWaves) void vsmall_kernel(V3Gemm g) {
     __syncthreads();
     for (int u = wave; u < MT * 4; u += W) {  // row slot u = 4 mt + r
         const int row = m0 + 16 * (u / 4) + 4 * j + u % 4;
-        if (row >= g.M) continue;
-        float v[NT];
+        if (row >= v.M) continue;
+        float x[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             float s = red[(u * NT + t) * kWave + lane];
             for (int w = 1; w < W; w++) s += red[((w * MT * 4 + u) * NT + t) * kWave + lane];
-            v[t] = s;
+            x[t] = s;
         }
-        v3_epi<EPI, NT>(g, sg, sstart, row, col, v, z);
+        v3_epi<WF, EPI, NT>(v, row, col, x, z);
     }
 }
 
 // ---- many rows ------------------------------------------------------------------------
 // Workgroup tile of BM rows x 16 WN NT weight columns, K in stages of 64 through one LDS
-// buffer (the next stage's global loads are in registers while this one computes; two or
+// buffer (the next AHEAD stages' global loads are in registers while this one computes; two or
 // three workgroups share a CU and cover each other's barriers).  4 waves in a WM x WN grid;
 // wave (wm, wn) owns the rows BM / WM of wm and the column tiles wn, wn + WN, ..., so that a
-// rotary pair (32 columns apart) and a gate / up pair lie in one lane.  LDS rows are 64
-// values (128 bytes) with their 16-byte chunks permuted by the row (chunk ^ row % 8): the 16
-// rows of a fragment read then fall in distinct banks without padding.
+// rotary pair (32 columns apart) and a gate / up pair lie in one lane.  The activations keep
+// their operand order in LDS; a weight row is 64 values (128 bytes) with its 16-byte chunks
+// permuted by the row (chunk ^ row % 8): the 16 rows of a fragment read then fall in distinct
+// banks without padding.
 template <int WF, int EPI, int BM, int WM, int NT>
-__global__ __launch_bounds__(256) void vtile_kernel(V3Gemm g) {
+__global__ __launch_bounds__(256, 2) void vtile_kernel(V3Gemm g) {
     constexpr int WN = 4 / WM, MT = BM / WM / 16, BN = 16 * WN * NT;
     constexpr bool DUAL = EPI == VE_SWIGLU;
+    constexpr int AHEAD = NT > 2 ? 1 : 2;   // stages in flight in registers (the wide tile has room for one)
     constexpr int CB = DUAL ? BN / 2 : BN;  // output columns per workgroup
     constexpr int AL = 3 * BM * 8 / 256, WL = WF == VW_Q4 ? (BN * 2 + 255) / 256 : BN * 8 / 256;
     static_assert(AL * 256 == 3 * BM * 8 && BN % 32 == 0, "whole chunks per thread");
@@ -300,79 +409,74 @@ __global__ __launch_bounds__(256) void vtile_kernel(V3Gemm g) {
     }
     if (bx >= gx) return;
     const int n0 = bx * CB, m0 = by * BM;
-    int sstart;
-    const VSeg& sg = g.seg[v3_seg_of(g, n0, sstart)];
-    const int G = g.K / 64, per = (G + g.ks - 1) / g.ks, s0 = z * per, S = min(G, s0 + per) - s0;
+    const V3View<WF, EPI> v = load_view<WF, EPI>(g, n0);
+    const int G = v.K / 64, per = (G + g.ks - 1) / g.ks, s0 = z * per, S = min(G, s0 + per) - s0;
     const uint16_t* ag[AL];
 #pragma unroll
     for (int i = 0; i < AL; i++) {
-        const int q = tid + 256 * i, p = q / (BM * 8), row = q / 8 % BM;
-        ag[i] = g.a + p * g.aps + (size_t)min(m0 + row, g.M - 1) * g.K + 8 * (q % 8);
+        // chunk q = [plane][row tile][k32 of the stage][lane]
+        const int q = tid + 256 * i, p = q / (BM * 8), mt = q / 128 % (BM / 16);
+        ag[i] = v.a + p * v.aps + (size_t)min(m0 / 16 + mt, (v.M - 1) / 16) * (v.K / 32) * 512 + 8 * (q % 128);
     }
     // weight column k of the tile: its row in the segment (DUAL: the second half is the up weight)
-    auto wrow = [&](int k, const VSeg*& s) {
-        s = DUAL && k >= CB ? &g.up : &sg;
-        return (size_t)min(n0 - sstart + (DUAL ? k % CB : k), s->n - 1);
+    auto wrow = [&](int k, bool& up) {
+        up = DUAL && k >= CB;
+        return (size_t)min(n0 - v.start + (DUAL ? k % CB : k), v.n - 1);
     };
     const char* wg[WL];
     const uint16_t *sr = nullptr, *br = nullptr;
     const bool wload = WF != VW_Q4 || tid < 2 * BN, sload = tid < BN;
 #pragma unroll
     for (int i = 0; i < WL; i++) {
-        const VSeg* s;
+        bool up;
         const int q = tid + 256 * i;
-        if (WF == VW_Q4) {
-            const size_t n = wrow(min(q / 2, BN - 1), s);
-            wg[i] = static_cast<const char*>(s->w) + n * (g.K / 2) + 16 * (q % 2);
-        } else {
-            const size_t n = wrow(q / 8, s);
-            wg[i] = static_cast<const char*>(s->w) + n * g.K * 2 + 16 * (q % 8);
-        }
+        const size_t n = wrow(WF == VW_Q4 ? min(q / 2, BN - 1) : q / 8, up);
+        wg[i] = (up ? v.wu : v.w) + (WF == VW_Q4 ? n * (v.K / 2) + 16 * (q % 2) : n * v.K * 2 + 16 * (q % 8));
     }
     if (WF == VW_Q4) {
-        const VSeg* s;
-        const size_t n = wrow(min(tid, BN - 1), s);
-        sr = s->s + n * G;
-        br = s->b + n * G;
+        bool up;
+        const size_t n = wrow(min(tid, BN - 1), up);
+        sr = (up ? v.su : v.s) + n * G;
+        br = (up ? v.bu : v.b) + n * G;
     }
-    uint4 ra[AL], rw[WL];
-    uint16_t rs = 0, rbi = 0;
-    auto gload = [&](int s) {
+    struct Stage {
+        uint4 a[AL], w[WL];
+        uint16_t s, b;
+    };
+    auto gload = [&](int s, Stage& r) {
         const int u = s0 + s;
 #pragma unroll
-        for (int i = 0; i < AL; i++) ra[i] = ldg4(ag[i] + 64 * (size_t)u);
+        for (int i = 0; i < AL; i++) r.a[i] = ldg4(ag[i] + 1024 * (size_t)u);
         if (wload)
 #pragma unroll
-            for (int i = 0; i < WL; i++) rw[i] = ldg4(wg[i] + (WF == VW_Q4 ? 32 : 128) * (size_t)u);
+            for (int i = 0; i < WL; i++) r.w[i] = ldg4(wg[i] + (WF == VW_Q4 ? 32 : 128) * (size_t)u);
         if (WF == VW_Q4 && sload) {
-            rs = gld(sr + u);
-            rbi = gld(br + u);
+            r.s = gld(sr + u);
+            r.b = gld(br + u);
         }
     };
-    auto lstore = [&]() {
+    const uint32_t mask = in_reg(kQ16Mask), magic = in_reg(kQ16Magic);
+    auto lstore = [&](const Stage& r) {
 #pragma unroll
-        for (int i = 0; i < AL; i++) {
-            const int q = tid + 256 * i, r = q / 8;  // r % BM = row: BM is a multiple of 8
-            As[r * 8 + ((q % 8) ^ (r % 8))] = ra[i];
-        }
+        for (int i = 0; i < AL; i++) As[tid + 256 * i] = r.a[i];
         if (WF == VW_Q4) {
             if (wload)
 #pragma unroll
                 for (int i = 0; i < WL; i++) {
                     const int q = tid + 256 * i, k = q / 2;
-                    const uint32_t e[4] = {rw[i].x, rw[i].y, rw[i].z, rw[i].w};
+                    const uint32_t e[4] = {r.w[i].x, r.w[i].y, r.w[i].z, r.w[i].w};
 #pragma unroll
-                    for (int w = 0; w < 4; w++) Ws[k * 8 + ((4 * (q % 2) + w) ^ (k % 8))] = unpack_q8(e[w]);
+                    for (int w = 0; w < 4; w++) Ws[k * 8 + ((4 * (q % 2) + w) ^ (k % 8))] = unpack_q16(e[w], mask, magic);
                 }
             if (sload) {
-                const float s = bf2f(rs);
-                Ss[tid] = make_float2(s, fmaf(8.0f, s, bf2f(rbi)));
+                const float s = bf2f(r.s);
+                Ss[tid] = make_float2(s, fmaf(-16.0f, s, bf2f(r.b)));
             }
         } else {
 #pragma unroll
             for (int i = 0; i < WL; i++) {
                 const int q = tid + 256 * i, k = q / 8;
-                Ws[k * 8 + ((q % 8) ^ (k % 8))] = rw[i];
+                Ws[k * 8 + ((q % 8) ^ (k % 8))] = r.w[i];
             }
         }
     };
@@ -382,36 +486,31 @@ __global__ __launch_bounds__(256) void vtile_kernel(V3Gemm g) {
 #pragma unroll
         for (int t = 0; t < NT; t++) hi[mt][t] = lo[mt][t] = kZero4;
     const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
-    auto afrag = [&](int p, int mt, int h) {
-        const int r = p * BM + wm * (BM / WM) + 16 * mt + c;
-        return As[r * 8 + ((4 * h + j) ^ (r % 8))];
-    };
+    auto afrag = [&](int p, int mt, int h) { return As[((p * (BM / 16) + wm * MT + mt) * 2 + h) * 64 + lane]; };
     auto wfrag = [&](int t, int h) {
         const int k = 16 * (t * WN + wn) + c;
         return Ws[k * 8 + ((4 * h + j) ^ (k % 8))];
     };
     auto compute = [&]() {
         if constexpr (WF == VW_Q4) {
-            f32x4_t th[MT][NT], tl[MT][NT], xh[MT], xl[MT];
+            f32x4_t th[MT][NT], xs[MT];
+            uint4 w[2][NT];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                uint4 w[NT];
+            for (int h = 0; h < 2; h++)
 #pragma unroll
-                for (int t = 0; t < NT; t++) w[t] = wfrag(t, h);
+                for (int t = 0; t < NT; t++) w[h][t] = wfrag(t, h);
 #pragma unroll
-                for (int p = 0; p < 3; p++)
+            for (int p = 2; p >= 0; p--)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
 #pragma unroll
                     for (int mt = 0; mt < MT; mt++) {
                         const uint4 a = afrag(p, mt, h);
-                        f32x4_t& x = p == 0 ? xh[mt] : xl[mt];
-                        x = mma(a, ones, h == 0 && p < 2 ? kZero4 : x);
+                        const bool first = p == 2 && h == 0;
+                        xs[mt] = mma(a, ones, first ? kZero4 : xs[mt]);
 #pragma unroll
-                        for (int t = 0; t < NT; t++) {
-                            f32x4_t& acc = p == 0 ? th[mt][t] : tl[mt][t];
-                            acc = mma(a, w[t], h == 0 && p < 2 ? kZero4 : acc);
-                        }
+                        for (int t = 0; t < NT; t++) th[mt][t] = mma(a, w[h][t], first ? kZero4 : th[mt][t]);
                     }
-            }
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 const float2 f = Ss[16 * (t * WN + wn) + c];
@@ -419,8 +518,7 @@ __global__ __launch_bounds__(256) void vtile_kernel(V3Gemm g) {
                 for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        hi[mt][t][r] = fmaf(f.x, th[mt][t][r] + tl[mt][t][r],
-                                            fmaf(f.y, xh[mt][r] + xl[mt][r], hi[mt][t][r]));
+                        hi[mt][t][r] = fmaf(f.x, th[mt][t][r], fmaf(f.y, xs[mt][r], hi[mt][t][r]));
             }
         } else {
 #pragma unroll
@@ -442,13 +540,32 @@ __global__ __launch_bounds__(256) void vtile_kernel(V3Gemm g) {
             }
         }
     };
-    if (S > 0) gload(0);
-    for (int s = 0; s < S; s++) {
-        lstore();
-        lds_sync();
-        if (s + 1 < S) gload(s + 1);
-        compute();
-        lds_sync();
+    Stage r0{};
+    if (S > 0) gload(0, r0);
+    if constexpr (AHEAD == 1) {
+        for (int s = 0; s < S; s++) {
+            lstore(r0);
+            lds_sync();
+            if (s + 1 < S) gload(s + 1, r0);
+            compute();
+            lds_sync();
+        }
+    } else {
+        Stage r1{};
+        if (S > 1) gload(1, r1);
+        for (int s = 0; s < S; s += 2) {
+            lstore(r0);
+            lds_sync();
+            if (s + 2 < S) gload(s + 2, r0);
+            compute();
+            lds_sync();
+            if (s + 1 >= S) break;
+            lstore(r1);
+            lds_sync();
+            if (s + 3 < S) gload(s + 3, r1);
+            compute();
+            lds_sync();
+        }
     }
     int col[NT];
 #pragma unroll
@@ -458,11 +575,11 @@ __global__ __launch_bounds__(256) void vtile_kernel(V3Gemm g) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int row = m0 + wm * (BM / WM) + 16 * mt + 4 * j + r;
-            if (row >= g.M) continue;
-            float v[NT];
+            if (row >= v.M) continue;
+            float x[NT];
 #pragma unroll
-            for (int t = 0; t < NT; t++) v[t] = hi[mt][t][r] + lo[mt][t][r];
-            v3_epi<EPI, NT>(g, sg, sstart, row, col, v, z);
+            for (int t = 0; t < NT; t++) x[t] = hi[mt][t][r] + lo[mt][t][r];
+            v3_epi<WF, EPI, NT>(v, row, col, x, z);
         }
 }
 
@@ -470,7 +587,7 @@ __global__ __launch_bounds__(256) void vtile_kernel(V3Gemm g) {
 // One workgroup per row: the row's values (SRC 0: the residual plus the K-slice partials in
 // slice order; SRC 1: the upsampled fc1 rows), stored as the next layer input, then
 // fast::rms_norm (w * (x * rsqrt(mean x^2 + eps))) into the planes of the next linear's
-// input.  NC = 16-byte chunks a thread holds in registers (0: any width, the row read back).
+// input.  NC = 8-value chunks a thread holds in registers (0: any width, the row read back).
 __device__ __forceinline__ float fc1_value(const VRowArgs& a, int r, int c) {
     // the fc1 row is bf16(acc + bias) for bf16 weights (addmm, one rounding) and
     // bf16(bf16(acc) + bias) for 4-bit ones (quantized_matmul, then the bias add)
@@ -479,64 +596,78 @@ __device__ __forceinline__ float fc1_value(const VRowArgs& a, int r, int c) {
 }
 
 template <int SRC, int NC>
-__global__ __launch_bounds__(256) void vrow_kernel(VRowArgs a) {
-    __shared__ float red[4];
-    const int m = blockIdx.x, N = a.N, n4 = N / 4, t = threadIdx.x;
+__global__ __launch_bounds__(128) void vrow_kernel(VRowArgs a) {
+    __shared__ float red[2];
+    const int m = blockIdx.x, N = a.N, n8 = N / 8, t = threadIdx.x;
+    struct V8 {
+        float e[8];
+    };
+    auto load8 = [&](const float* p) {
+        const float4 x = reinterpret_cast<const float4*>(p)[0], y = reinterpret_cast<const float4*>(p)[1];
+        return V8{{x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w}};
+    };
     // Decoder._linear_upsample_1d (align_corners=False, f32)
     const float pos = ((float)m + 0.5f) / (float)a.scale - 0.5f;
     const int left = (int)floorf(pos);
     const float wr = pos - (float)left, wl = 1.0f - wr;
     const int l = min(max(left, 0), a.T - 1), r = min(max(left + 1, 0), a.T - 1);
     auto value = [&](int i) {
-        float4 x;
+        V8 x;
         if constexpr (SRC == 1) {
-            float e[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) e[k] = fc1_value(a, l, 4 * i + k) * wl + fc1_value(a, r, 4 * i + k) * wr;
-            x = make_float4(e[0], e[1], e[2], e[3]);
+            for (int k = 0; k < 8; k++) x.e[k] = fc1_value(a, l, 8 * i + k) * wl + fc1_value(a, r, 8 * i + k) * wr;
         } else {
-            float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            x = load8(a.res + (size_t)m * N + 8 * i);
+            V8 s{};
             for (int z = 0; z < a.ks; z++) {
-                const float4 p = reinterpret_cast<const float4*>(a.part + ((size_t)z * a.M + m) * N)[i];
-                s = make_float4(s.x + p.x, s.y + p.y, s.z + p.z, s.w + p.w);
+                const V8 p = load8(a.part + ((size_t)z * a.M + m) * N + 8 * i);
+#pragma unroll
+                for (int k = 0; k < 8; k++) s.e[k] += p.e[k];
             }
-            const float4 q = reinterpret_cast<const float4*>(a.res + (size_t)m * N)[i];
-            x = make_float4(q.x + s.x, q.y + s.y, q.z + s.z, q.w + s.w);
+#pragma unroll
+            for (int k = 0; k < 8; k++) x.e[k] += s.e[k];
         }
-        reinterpret_cast<float4*>(a.x + (size_t)m * N)[i] = x;
+        float4* o = reinterpret_cast<float4*>(a.x + (size_t)m * N + 8 * i);
+        o[0] = make_float4(x.e[0], x.e[1], x.e[2], x.e[3]);
+        o[1] = make_float4(x.e[4], x.e[5], x.e[6], x.e[7]);
         return x;
     };
-    float4 xv[NC > 0 ? NC : 1];
+    V8 xv[NC > 0 ? NC : 1];
     float ss = 0.0f;
-    auto sq = [&](const float4& x) { ss += (x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w); };
+    auto sq = [&](const V8& x) {
+#pragma unroll
+        for (int k = 0; k < 8; k += 4)
+            ss += (x.e[k] * x.e[k] + x.e[k + 1] * x.e[k + 1]) + (x.e[k + 2] * x.e[k + 2] + x.e[k + 3] * x.e[k + 3]);
+    };
     if constexpr (NC > 0) {
 #pragma unroll
         for (int k = 0; k < NC; k++)
-            if (t + 256 * k < n4) {
-                xv[k] = value(t + 256 * k);
+            if (t + 128 * k < n8) {
+                xv[k] = value(t + 128 * k);
                 sq(xv[k]);
             }
     } else {
-        for (int i = t; i < n4; i += 256) sq(value(i));
+        for (int i = t; i < n8; i += 128) sq(value(i));
     }
     ss = block_sum(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float)N + a.eps);
-    auto put = [&](int i, const float4& x) {
-        const float e[4] = {x.x, x.y, x.z, x.w};
-        uint32_t p[4][3];
+    auto put = [&](int i, const V8& x) {
+        uint32_t p[8][3];
 #pragma unroll
-        for (int k = 0; k < 4; k++) split3(bf2f(gld(a.w + 4 * i + k)) * (e[k] * inv), p[k]);
+        for (int k = 0; k < 8; k++) split3(bf2f(gld(a.w + 8 * i + k)) * (x.e[k] * inv), p[k]);
 #pragma unroll
-        for (int q = 0; q < 3; q++)
-            *reinterpret_cast<uint2*>(a.h + q * a.hps + (size_t)m * N + 4 * i) =
-                make_uint2(hi_pair(p[0][q], p[1][q]), hi_pair(p[2][q], p[3][q]));
+        for (int q = 0; q < 3; q++) {
+            const uint4 v = make_uint4(hi_pair(p[0][q], p[1][q]), hi_pair(p[2][q], p[3][q]), hi_pair(p[4][q], p[5][q]),
+                                       hi_pair(p[6][q], p[7][q]));
+            *reinterpret_cast<uint4*>(a.h + q * a.hps + plane_at(m, 8 * i, N, 0)) = a.hpair ? pair_order(v) : v;
+        }
     };
     if constexpr (NC > 0) {
 #pragma unroll
         for (int k = 0; k < NC; k++)
-            if (t + 256 * k < n4) put(t + 256 * k, xv[k]);
+            if (t + 128 * k < n8) put(t + 128 * k, xv[k]);
     } else {
-        for (int i = t; i < n4; i += 256) put(i, reinterpret_cast<const float4*>(a.x + (size_t)m * N)[i]);
+        for (int i = t; i < n8; i += 128) put(i, load8(a.x + (size_t)m * N + 8 * i));
     }
 }
 
@@ -549,7 +680,7 @@ __global__ __launch_bounds__(256) void vrow_kernel(VRowArgs a) {
 // over the banks.  The row leaves as the planes of the o projection's input.
 constexpr int kVKs = 68;
 __global__ __launch_bounds__(1024) void vattn_gqa_kernel(const float* qkv, int M, int ldq, int H, int heads, int kvh,
-                                                         int window, float scale, uint16_t* att, size_t aps) {
+                                                         int window, float scale, uint16_t* att, size_t aps, int pair) {
     __shared__ __align__(16) float ks[64 * kVKs];
     __shared__ __align__(16) float vs[64 * 64];
     const int i = blockIdx.x / kvh, kh = blockIdx.x % kvh, grp = heads / kvh;
@@ -585,18 +716,22 @@ __global__ __launch_bounds__(1024) void vattn_gqa_kernel(const float* qkv, int M
     }
     uint32_t pl[3];
     split3(o / l, pl);
-    uint16_t* y = att + (size_t)i * H + h * 64 + lane;
+    uint16_t* y = att + plane_at(i, h * 64 + lane, H, pair);
 #pragma unroll
     for (int k = 0; k < 3; k++) gst(y + k * aps, (uint16_t)(pl[k] >> 16));
 }
 
+constexpr int kSmallTwoTiles = 128;
+
 template <int WF, int EPI, int NP>
 hipError_t launch_small(hipStream_t st, const V3Gemm& g, int N) {
-    constexpr int NT = EPI == VE_QKV || EPI == VE_SWIGLU ? 2 : 1;
+    constexpr int NT = kSmallNT<EPI>;
     const int per = (g.K / kUnitK<WF> + g.ks - 1) / g.ks;
-    const int W = min(kSmallWaves, (per + kSmallCh<WF> - 1) / kSmallCh<WF>);
-    const int gx = EPI == VE_QKV ? N / 32 : (N + 15) / 16;
-    const int mt = g.M > 16 ? 2 : 1;
+    const int W = min(kSmallWaves<EPI>, (per + kSmallCh<WF> - 1) / kSmallCh<WF>);
+    const int gx = EPI == VE_QKV ? N / 32 : (EPI == VE_SWIGLU ? N / 32 : (N + 15) / 16);
+    // two row tiles per workgroup share its weights; with few column blocks one each, so that
+    // twice the CUs pull the activations
+    const int mt = g.M > 16 && gx * g.ks >= kSmallTwoTiles ? 2 : 1;
     const dim3 grid(gx, (g.M + 16 * mt - 1) / (16 * mt), g.ks);
     const size_t lds = sizeof(float) * (size_t)W * mt * 4 * NT * kWave;
     if (mt == 2)
@@ -656,29 +791,29 @@ hipError_t launch_v3gemm(hipStream_t st, const V3Gemm& g, int wf, int epi) {
 }
 
 hipError_t launch_vrow(hipStream_t st, const VRowArgs& a, bool upsample) {
-    if (a.N % 4 || a.N < 4 || a.M < 1) return hipErrorInvalidValue;
+    if (a.N % 32 || a.N < 32 || a.M < 1) return hipErrorInvalidValue;
     const bool one = a.N <= 1024;
     if (upsample) {
         if (one)
-            hipLaunchKernelGGL((vrow_kernel<1, 1>), dim3(a.M), dim3(256), 0, st, a);
+            hipLaunchKernelGGL((vrow_kernel<1, 1>), dim3(a.M), dim3(128), 0, st, a);
         else
-            hipLaunchKernelGGL((vrow_kernel<1, 0>), dim3(a.M), dim3(256), 0, st, a);
+            hipLaunchKernelGGL((vrow_kernel<1, 0>), dim3(a.M), dim3(128), 0, st, a);
     } else {
         if (one)
-            hipLaunchKernelGGL((vrow_kernel<0, 1>), dim3(a.M), dim3(256), 0, st, a);
+            hipLaunchKernelGGL((vrow_kernel<0, 1>), dim3(a.M), dim3(128), 0, st, a);
         else
-            hipLaunchKernelGGL((vrow_kernel<0, 0>), dim3(a.M), dim3(256), 0, st, a);
+            hipLaunchKernelGGL((vrow_kernel<0, 0>), dim3(a.M), dim3(128), 0, st, a);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_vattn(hipStream_t st, const float* qkv, int M, int ldq, int H, int heads, int kvh, int window,
-                        float scale, uint16_t* att, size_t aps) {
+                        float scale, uint16_t* att, size_t aps, int pair) {
     if (window < 1 || window > 64 || kvh < 1 || heads % kvh) return hipErrorInvalidValue;
     const int grp = heads / kvh;
     if (grp > 16) return hipErrorInvalidValue;  // rejected at model creation
     hipLaunchKernelGGL(vattn_gqa_kernel, dim3(M * kvh), dim3(64 * grp), 0, st, qkv, M, ldq, H, heads, kvh, window,
-                       scale, att, aps);
+                       scale, att, aps, pair);
     return hipGetLastError();
 }
 

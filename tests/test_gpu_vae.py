@@ -114,3 +114,40 @@ def test_vae_rejects(ming, ctx):
     with pytest.raises(ming.MingError) as e:
         ming.VaeModel(ctx, c, syn.w, 4)
     assert e.value.status == ming.MING_E_UNSUPPORTED
+
+
+@pytest.mark.parametrize("rows, quant, over", [
+    (16, False, {}), (17, True, {}), (64, False, dict(inter=1152)),  # unstaged kernel: one tile, a remainder, K slices
+    (65, True, dict(inter=1152)), (133, False, dict(inter=2176)),    # LDS tiles: a remainder, K slices of unequal length
+    (257, True, dict(hidden=256, heads=4, kv_heads=2)),
+])
+def test_vae_row_counts(ming, ctx, rows, quant, over):
+    """Either side of the row-count rules of the linears (16, 32, 64 rows) and of their K slices; the bars
+    are those of check()."""
+    S = syn_mod()
+    syn = S.SyntheticVae(ctx, S.VaeSpec(**dict(SMALL, patch=1, **over)), seed=27, quant=quant, std=0.05, norm_std=0.1)
+    check(ming, ctx, syn, rows)
+
+
+@pytest.mark.parametrize("hop", [1, 6, 35, 11, 13 * 5])
+def test_vae_transform_lengths(ming, ctx, hop):
+    """ISTFT by FFT passes (n_fft / 2 = 2, 12, 70: every radix, an odd one last) and by the basis GEMM (a prime
+    factor above 7)."""
+    S = syn_mod()
+    syn = S.SyntheticVae(ctx, S.VaeSpec(**dict(SMALL, n_fft=4 * hop, hop=hop)), seed=28, std=0.05, norm_std=0.1)
+    check(ming, ctx, syn, 5)
+
+
+def test_vae_latents_off_alignment(ming, ctx):
+    """Latents 2 bytes off a 16-byte boundary give the aligned call's bits."""
+    S = syn_mod()
+    syn = S.SyntheticVae(ctx, S.VaeSpec(**SMALL), seed=29, std=0.05)
+    m = syn.model(7)
+    buf = torch.empty(7 * 64 + 8, dtype=torch.bfloat16, device="cuda").normal_()
+    waves = []
+    for lat in (buf[1:1 + 7 * 64], buf[1:1 + 7 * 64].clone()):
+        waves.append(torch.empty(7 * 4 * 16, dtype=torch.float32, device="cuda"))
+        m.decode(7, lat, waves[-1])
+    ctx.sync()
+    m.close()
+    assert torch.equal(waves[0], waves[1])
