@@ -688,46 +688,61 @@ int ming_cfm_sample_batch(ming_ctx* ctx, ming_cfm_model* m, int32_t n, const voi
     auto grow = [&](DevBuf& d, size_t bytes) {
         if (e == hipSuccess) e = d.ensure(bytes);
     };
+    const bool flow = flow_block_fits(D, F, m->cfg.head_dim, lat);
+    const size_t Rp = ((size_t)R + 15) / 16 * 16;  // operand-order buffers hold whole row tiles
     grow(m->bce, (size_t)n * D * b2);
     grow(m->bxh, (size_t)n * D * b2);
-    grow(m->bxe, (size_t)n * D * b2);
     grow(m->brows[0], (size_t)R * D * b2);
     grow(m->brows[1], (size_t)R * D * b2);
-    grow(m->bhn, (size_t)R * D * b2);
-    grow(m->bqkv, (size_t)3 * R * D * b2);
-    grow(m->batt, (size_t)R * D * b2);
+    grow(m->batt, Rp * D * b2);
     grow(m->bx1, (size_t)R * D * b2);
-    grow(m->bhh, (size_t)R * F * b2);
+    grow(m->bhh, Rp * F * b2);
     grow(m->by[0], (size_t)n * lat * b2);
     grow(m->by[1], (size_t)n * lat * b2);
-    grow(m->bhf, (size_t)2 * n * D * b2);
-    grow(m->bpart, (size_t)R * std::max(4 * D, 2 * F) * sizeof(float));  // split-K partials of ff2 / ff1
+    if (!flow) {
+        grow(m->bxe, (size_t)n * D * b2);
+        grow(m->bhn, (size_t)R * D * b2);
+        grow(m->bqkv, (size_t)3 * R * D * b2);
+        grow(m->bhf, (size_t)2 * n * D * b2);
+        grow(m->bpart, (size_t)R * std::max(4 * D, 2 * F) * sizeof(float));  // split-K partials of ff2 / ff1
+    }
     if (e != hipSuccess) return hip_check(ctx, e, "cfm_sample_batch workspace");
     const float eps = m->cfg.eps;
     // once per sample: c_emb(z) (the unconditional half is c_emb(0) = bias) and x_emb(hist) (:1196-1197)
     e = launch_dit_linear_gemm(s, u16(z), n, m->wc, D, H, m->bc, u16(m->bce.p));
     if (e == hipSuccess) e = launch_dit_linear_gemm(s, u16(hist), n, m->wx, D, lat, m->bx, u16(m->bxh.p));
     const uint16_t* y = u16(noise);
+    const float *cos_t = static_cast<const float*>(m->cos.p), *sin_t = static_cast<const float*>(m->sin.p);
     int yi = 0;
     for (int i = 0; i < kFlowSteps && e == hipSuccess; i++) {
-        e = launch_dit_linear_gemm(s, y, n, m->wx, D, lat, m->bx, u16(m->bxe.p));
-        if (e == hipSuccess)
-            e = launch_cfm_rows_batch(s, u16(m->t_emb.p) + (size_t)i * 2 * D, u16(m->bce.p), m->bc, u16(m->bxh.p),
-                                      u16(m->bxe.p), n, D, u16(m->brows[0].p));
+        const uint16_t* te = u16(m->t_emb.p) + (size_t)i * 2 * D;
         int cur = 0;
-        for (size_t bl = 0; bl < m->blocks.size() && e == hipSuccess; bl++) {
-            // each block leaves the next one's rms1 of its output in bhn (fused into its ff2 reduce)
-            e = launch_dit_block_gemm(s, m->blocks[bl], u16(m->brows[cur].p), R, L,
-                                      static_cast<const float*>(m->cos.p), static_cast<const float*>(m->sin.p),
-                                      u16(m->bhn.p), u16(m->bqkv.p), u16(m->batt.p), u16(m->bx1.p), u16(m->bhh.p),
-                                      u16(m->brows[cur ^ 1].p), static_cast<float*>(m->bpart.p), bl > 0,
-                                      bl + 1 < m->blocks.size() ? &m->blocks[bl + 1] : nullptr);
-            cur ^= 1;
+        if (flow) {
+            e = launch_flow_rows(s, y, lat, m->wx, m->bx, te, u16(m->bce.p), m->bc, u16(m->bxh.p), n, D,
+                                 u16(m->brows[0].p));
+            for (size_t bl = 0; bl < m->blocks.size() && e == hipSuccess; bl++, cur ^= 1)
+                e = launch_flow_block(s, m->blocks[bl], u16(m->brows[cur].p), R, cos_t, sin_t, u16(m->batt.p),
+                                      u16(m->bx1.p), u16(m->bhh.p), u16(m->brows[cur ^ 1].p));
+            if (e == hipSuccess)
+                e = launch_flow_final(s, u16(m->brows[cur].p), n, D, m->final_norm, eps, m->wf, m->bf, lat, y,
+                                      u16(m->dtd.p), u16(m->sqd.p), u16(sde), i, kFlowSteps, cfg, shift,
+                                      u16(m->by[yi].p), u16(y_steps));
+        } else {
+            e = launch_dit_linear_gemm(s, y, n, m->wx, D, lat, m->bx, u16(m->bxe.p));
+            if (e == hipSuccess)
+                e = launch_cfm_rows_batch(s, te, u16(m->bce.p), m->bc, u16(m->bxh.p), u16(m->bxe.p), n, D,
+                                          u16(m->brows[0].p));
+            for (size_t bl = 0; bl < m->blocks.size() && e == hipSuccess; bl++, cur ^= 1)
+                // each block leaves the next one's rms1 of its output in bhn (fused into its ff2 reduce)
+                e = launch_dit_block_gemm(s, m->blocks[bl], u16(m->brows[cur].p), R, L, cos_t, sin_t, u16(m->bhn.p),
+                                          u16(m->bqkv.p), u16(m->batt.p), u16(m->bx1.p), u16(m->bhh.p),
+                                          u16(m->brows[cur ^ 1].p), static_cast<float*>(m->bpart.p), bl > 0,
+                                          bl + 1 < m->blocks.size() ? &m->blocks[bl + 1] : nullptr);
+            if (e == hipSuccess)
+                e = launch_cfm_final_batch(s, u16(m->brows[cur].p), n, L, D, m->final_norm, eps, m->wf, m->bf, lat, y,
+                                           u16(m->dtd.p), u16(m->sqd.p), u16(sde), i, kFlowSteps, cfg, shift,
+                                           u16(m->bhf.p), u16(m->by[yi].p), u16(y_steps));
         }
-        if (e == hipSuccess)
-            e = launch_cfm_final_batch(s, u16(m->brows[cur].p), n, L, D, m->final_norm, eps, m->wf, m->bf, lat, y,
-                                       u16(m->dtd.p), u16(m->sqd.p), u16(sde), i, kFlowSteps, cfg, shift,
-                                       u16(m->bhf.p), u16(m->by[yi].p), u16(y_steps));
         y = u16(m->by[yi].p);
         yi ^= 1;
     }

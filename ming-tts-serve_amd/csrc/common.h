@@ -44,8 +44,6 @@ __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
 // is 0 (e^-86 < 2^-124; the scaled polynomial would reach denormals), above 88
 // +inf; NaN stays NaN.
 __device__ __forceinline__ float exp_rep(float x) {
-    if (x < -86.0f) return 0.0f;
-    if (x > 88.0f) return __builtin_inff();
     const float n = __builtin_rintf(x * 0x1.715476p+0f);
     float r = __builtin_fmaf(n, -0x1.62e4p-1f, x);
     r = __builtin_fmaf(n, -0x1.7f7d1cp-20f, r);
@@ -57,7 +55,8 @@ __device__ __forceinline__ float exp_rep(float x) {
     p = __builtin_fmaf(p, r, 0.5f);
     p = __builtin_fmaf(p, r, 1.0f);
     p = __builtin_fmaf(p, r, 1.0f);
-    return __builtin_ldexpf(p, (int)n);
+    const float e = __builtin_ldexpf(p, (int)n);
+    return x < -86.0f ? 0.0f : (x > 88.0f ? __builtin_inff() : e);  // selects: no branch per value
 }
 
 // acc + a.lo*b.lo + a.hi*b.hi with bf16 pairs packed in u32 (v_dot2c_f32_bf16).

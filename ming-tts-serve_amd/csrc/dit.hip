@@ -29,6 +29,7 @@
 #include <mutex>
 #include <vector>
 
+#include "dit_attn.h"
 #include "gemv.h"
 #include "internal.h"
 #include "tanh_tab.h"
@@ -41,7 +42,6 @@ constexpr int kMaxR = 6;       // activation rows of a reference-shape block (2 
 constexpr int kMaxSlots = 20;  // row slots of the widest launch (adaLN modulations: 10 steps x 2 halves)
 // 16-byte LDS vector (the staged rows are 16-byte aligned: K % 8 == 0)
 typedef uint32_t lds_u32x4_t __attribute__((ext_vector_type(4), aligned(16)));
-constexpr int kMaxL = 8;  // positions per sequence (attention)
 constexpr int kMaxH = 4;  // heads per wave in dit_attn_out_kernel (16 heads, 4 waves)
 
 enum DitEpi {
@@ -483,36 +483,6 @@ __global__ __launch_bounds__(256) void adaln_cond_kernel(const uint16_t* te, con
     const float v = rb(bf2f(gld(te + i)) + bf2f(gld(ce + i % (2 * D))));
     const float sg = rb(1.0f / (1.0f + exp_rep(-v)));
     gst(out + i, f2bf(v * sg));
-}
-
-// Attention of one (sequence, head) over its L positions on the wave, lane d
-// holding dimension d of q, k and v (lanes past head_dim: on = false, adding
-// zeros): scores sum_d (q/8) k in f32 (wave sums), p = exp(s - max),
-// l = sum p, o[i] = (sum_j p_j v_j) / l, to be rounded once by the caller.
-__device__ __forceinline__ void attn_math(const float (&qv)[kMaxL], const float (&kv)[kMaxL],
-                                          const float (&vv)[kMaxL], int L, bool on, float (&o)[kMaxL]) {
-    const float scale = 1.0f / 8.0f;
-#pragma unroll
-    for (int i = 0; i < kMaxL; i++)
-        if (i < L) {
-            const float qd = on ? scale * qv[i] : 0.0f;
-            float sc[kMaxL], m = -INFINITY;
-#pragma unroll
-            for (int j = 0; j < kMaxL; j++)
-                if (j < L) {
-                    sc[j] = team_sum<kWave>(qd * kv[j]);
-                    m = fmaxf(m, sc[j]);
-                }
-            float l = 0.0f, acc = 0.0f;
-#pragma unroll
-            for (int j = 0; j < kMaxL; j++)
-                if (j < L) {
-                    const float p = exp_rep(sc[j] - m);
-                    l += p;
-                    acc += p * vv[j];
-                }
-            o[i] = acc / l;
-        }
 }
 
 // Attention over the L positions of each sequence, one wave per (sequence,

@@ -128,6 +128,17 @@ hipError_t launch_cfm_final_batch(hipStream_t st, const uint16_t* h, int n, int 
                                   const uint16_t* dt, const uint16_t* sq, const uint16_t* sde, int step, int steps,
                                   float cfg, float shift, uint16_t* hn, uint16_t* y_out, uint16_t* y_steps);
 
+bool flow_block_fits(int D, int F, int hd, int latent);
+hipError_t launch_flow_block(hipStream_t st, const DitBlockDev& w, const uint16_t* x, int R, const float* cos_t,
+                             const float* sin_t, uint16_t* att, uint16_t* x1, uint16_t* hh, uint16_t* out);
+hipError_t launch_flow_rows(hipStream_t st, const uint16_t* y, int lat, const uint16_t* wx, const uint16_t* bx,
+                            const uint16_t* te, const uint16_t* ce, const uint16_t* bc, const uint16_t* xh, int n,
+                            int D, uint16_t* rows);
+hipError_t launch_flow_final(hipStream_t st, const uint16_t* h, int n, int D, const uint16_t* norm, float eps,
+                             const uint16_t* wf, const uint16_t* bf, int latent, const uint16_t* y, const uint16_t* dt,
+                             const uint16_t* sq, const uint16_t* sde, int step, int steps, float cfg, float shift,
+                             uint16_t* y_out, uint16_t* y_steps);
+
 // Read-only view of a prepared decode stack (for the batched step).
 struct LmView {
     ming_lm_cfg cfg;

@@ -23,6 +23,13 @@ __device__ __forceinline__ float tanh_bf16(const float* __restrict__ tab, float 
     return (b & 0x8000u) ? -t : t;
 }
 
+// The same from an entry loaded beforehand: e = tab[min(m, kTanhTabN - 1)].
+__device__ __forceinline__ float tanh_bf16_of(float e, float u) {
+    const uint32_t b = __float_as_uint(u) >> 16, m = b & 0x7fffu;
+    const float t = m < (uint32_t)kTanhTabN ? e : (m > 0x7f80u ? u : 1.0f);
+    return (b & 0x8000u) ? -t : t;
+}
+
 // The table on the host (computed once).
 const float* tanh_table_host();
 

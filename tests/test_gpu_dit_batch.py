@@ -174,3 +174,48 @@ def test_cfm_batch_end_to_end_exact(ming, ctx, flowb, n, cfg, sigma, temperature
             for i in range(10):
                 assert_bits(gs[b, i], rsteps[i], f"sequence {b} free-running Euler step {i} (batched order)")
             assert_bits(g[b], ref, f"sequence {b} latent")
+
+
+@pytest.mark.parametrize("n", [2, 3, 8, 11, 21, 22, 40, 41, 43])
+def test_cfm_batch_row_tiles(ming, ctx, flowb, n):
+    """The tiles that 6 n rows take (1 to 24 row tiles of 16, 5 or 10 row groups a q/k/v workgroup, 1 to 3 row
+    tiles a workgroup of the other linears) and their remainders: the first and last sequences equal a
+    one-sequence call bit for bit."""
+    syn, m, _, _ = flowb
+    spec = syn.spec
+    z, hist, noise, sde = (dev_u16(a) for a in inputs(ming, spec, n, f"tile{n}"))
+    out = torch.empty((n, spec.latent), dtype=torch.bfloat16, device="cuda")
+    m.sample_batch(n, z, hist, noise, sde, 2.0, 0.25, 1.0, out)
+    one = torch.empty((1, spec.latent), dtype=torch.bfloat16, device="cuda")
+    for b in (0, n // 2, n - 1):
+        m.sample_batch(1, z[b:b + 1], hist[b:b + 1], noise[b:b + 1], sde[b:b + 1], 2.0, 0.25, 1.0, one)
+        ctx.sync()
+        assert torch.equal(one[0], out[b]), b
+
+
+@pytest.mark.parametrize("hidden,heads,ff", [(128, 2, 256), (512, 8, 1024), (512, 8, 2048), (1024, 16, 512),
+                                             (768, 12, 1536)])
+def test_cfm_batch_shapes(ming, ctx, hidden, heads, ff):
+    """Other shapes, bit for bit with the oracle in the batched kernels' order: the four-launch block (hidden 512 and
+    1024 with whole K slices of ff; one, two and four of them) and the general one (128, 768)."""
+    S = syn_mod()
+    spec = S.DitSpec(hidden=hidden, heads=heads, head_dim=64, ff=ff, cfm_blocks=2)
+    syn = S.SyntheticFlow(ctx, spec, seed=67, norm_std=0.05, parts=("cfm",))
+    m, n = syn.cfm_model(), 7
+    with oracle.dit_order(oracle.DIT_ORDER_DEVICE):
+        od = oracle_cfm(syn)
+    z, hist, noise, sde = inputs(ming, spec, n, f"shape{hidden}")
+    out = torch.empty((n, spec.latent), dtype=torch.bfloat16, device="cuda")
+    steps = torch.empty((n, 10, spec.latent), dtype=torch.bfloat16, device="cuda")
+    m.sample_batch(n, dev_u16(z), dev_u16(hist), dev_u16(noise), dev_u16(sde), 2.0, 0.25, 1.0, out, steps)
+    ctx.sync()
+    g = host_u16(steps)
+    with oracle.dit_order(oracle.DIT_ORDER_MFMA):
+        for b in (0, n - 1):
+            for i in (0, 9):
+                y_in = noise[b] if i == 0 else g[b, i - 1]
+                h = oracle.cfm_rows(od, z[b], hist[b], y_in, i)
+                for blk in od.blocks:
+                    h = oracle.dit_block_fwd(ocfg(spec), blk, h, 2, 3, od.keep["cos"], od.keep["sin"])
+                assert_bits(g[b, i], oracle.cfm_final(od, h, 3, y_in, sde[b], i, 2.0, 0.25),
+                            f"sequence {b} Euler step {i}")
