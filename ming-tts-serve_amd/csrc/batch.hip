@@ -283,6 +283,160 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(PagedAttnArgs a) {
     }
 }
 
+// ---- paged attention of a prompt's rows ---------------------------------------------------
+// Rows b of one sequence at consecutive positions (prefill): the MFMA columns are 16 rows of one
+// head, where the kernel above has one row's grp heads and reads the row's whole K and V for it.
+// Workgroup (split s, kv head g and head part, row tile): wave w holds page 4 s + w's K and V
+// operands and walks its part's heads; a column's arithmetic and the order in which the pages
+// meet are the kernel above's, bit for bit (a page past a row contributes m = -inf, l = o = 0).
+// A whole prompt reads its pages once per 16 rows: 512 rows at 1529 .. 2040 cached positions
+// took 65 us a layer one row at a time (1024 workgroups' K and V reads and 9 of 16 columns idle).
+__global__ __launch_bounds__(256) void prefill_attn_kernel(PagedAttnArgs a, int n, int hper) {
+    extern __shared__ uint4 qs[];  // [16 rows][hper * 8 + 1]: scaled q
+    __shared__ float so[2][4][16][64];
+    __shared__ float sm[2][4][16], sl[2][4][16];
+    const int s = blockIdx.x, hparts = (a.grp + hper - 1) / hper, g = blockIdx.y / hparts, h0 = blockIdx.y % hparts * hper,
+              h1 = min(h0 + hper, a.grp), r0 = blockIdx.z * 16;
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, c = lane % 16, j = lane / 16;
+    const int rl = min(r0 + 15, n - 1), row = min(r0 + c, n - 1);
+    const int plast = gld(a.pos + rl), pos = gld(a.pos + row);
+    if (plast < 0 || plast >= a.pages_per_seq * 64) {
+        if (tid == 0 && s == 0) gst(a.flags, 1);
+        return;
+    }
+    if (s * 256 > plast) return;
+    const int pi = 4 * s + wave, len = pos + 1, base = pi * 64;
+    bool any = base <= plast;
+    if (any) {
+        const int page = gld(a.table + (size_t)r0 * a.pages_per_seq + pi);
+        if (page < 0 || page >= a.n_pages) {
+            any = false;
+            if (lane == 0) gst(a.flags, 1);
+        }
+    }
+    uint4 ka[4][2], va[4][2];
+    if (any) {
+        const int page = gld(a.table + (size_t)r0 * a.pages_per_seq + pi);
+        const size_t pbase = ((size_t)page * a.kvh + g) * 64 * 64;
+        const uint16_t* kb = a.kp + pbase;
+        const uint16_t* vb = a.vp + pbase;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int p = 32 * (t / 2) + 8 * (c / 4) + 4 * (t % 2) + c % 4;
+            ka[t][0] = ldg4(kb + p * 64 + 16 * j);
+            ka[t][1] = ldg4(kb + p * 64 + 16 * j + 8);
+        }
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) va[dt][u] = ldg4(vb + (16 * dt + c) * 64 + 32 * u + 8 * j);
+    }
+    const int qc = (h1 - h0) * 8, qld = hper * 8 + 1;
+    for (int k = tid; k < 16 * qc; k += 256) {
+        const int r = k / qc, ch = k % qc;
+        const uint4 v = ldg4(a.qkv + (size_t)min(r0 + r, n - 1) * a.ldq + (g * a.grp + h0) * 64 + 8 * ch);
+        const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+        uint32_t r4[4];
+#pragma unroll
+        for (int p = 0; p < 4; p++) r4[p] = pack_bf2(bf_lo(e[p]) * a.scale, bf_hi(e[p]) * a.scale);
+        qs[r * qld + ch] = make_uint4(r4[0], r4[1], r4[2], r4[3]);
+    }
+    lds_sync();
+    const bool has = any && base < len;  // this lane's column
+    for (int h = h0; h < h1; h++) {
+        const int buf = (h - h0) & 1;
+        float mx = -INFINITY, l = 0.0f;
+        f32x4_t o[4];
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) o[dt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        if (any) {
+            const uint4 *qp = qs + c * qld + (h - h0) * 8 + 2 * j, q0 = qp[0], q1 = qp[1];
+            f32x4_t sc[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                sc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(ka[t][0]), as_bf8(q0), sc[t], 0, 0, 0);
+                sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(ka[t][1]), as_bf8(q1), sc[t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int p = 32 * (t / 2) + 8 * j + 4 * (t % 2) + r;
+                    if (base + p >= len) sc[t][r] = -INFINITY;
+                    mx = fmaxf(mx, sc[t][r]);
+                }
+            mx = rows_max(mx);
+            const float mz = has ? mx : 0.0f;
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float e = att_exp(sc[t][r] - mz);  // masked scores (-inf) give 0
+                    sc[t][r] = e;
+                    l += e;
+                }
+            l = rows_sum(l);
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float p0 = sc[2 * u + k / 2][2 * (k % 2)], p1 = sc[2 * u + k / 2][2 * (k % 2) + 1];
+                    hi[k] = pack_bf2(p0, p1);
+                    lo[k] = pack_bf2(p0 - bf_lo(hi[k]), p1 - bf_hi(hi[k]));
+                }
+                const bf16x8_t ph = as_bf8(make_uint4(hi[0], hi[1], hi[2], hi[3]));
+                const bf16x8_t pl = as_bf8(make_uint4(lo[0], lo[1], lo[2], lo[3]));
+#pragma unroll
+                for (int dt = 0; dt < 4; dt++) {
+                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(va[dt][u]), ph, o[dt], 0, 0, 0);
+                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(va[dt][u]), pl, o[dt], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) so[buf][wave][dt * 4 + r][lane] = has ? o[dt][r] : 0.0f;
+        if (j == 0) {
+            sm[buf][wave][c] = has ? mx : -INFINITY;
+            sl[buf][wave][c] = has ? l : 0.0f;
+        }
+        // one barrier a head: the wave that joins head h leaves it before its barrier of head h + 1,
+        // and buffer h is written again after that
+        lds_sync();
+        if (wave != (h & 3)) continue;
+        float M = sm[buf][0][c];
+#pragma unroll
+        for (int w = 1; w < 4; w++) M = fmaxf(M, sm[buf][w][c]);
+        float f[4], L = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            f[w] = sm[buf][w][c] == -INFINITY ? 0.0f : att_exp(sm[buf][w][c] - M);
+            L += f[w] * sl[buf][w][c];
+        }
+        if (r0 + c >= n || s * 256 >= len) continue;
+        float* pp = a.part + ((((size_t)(r0 + c) * a.kvh + g) * a.max_splits + s) * a.grp + h) * 68;
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                v[r] = f[0] * so[buf][0][dt * 4 + r][lane];
+#pragma unroll
+                for (int w = 1; w < 4; w++) v[r] += f[w] * so[buf][w][dt * 4 + r][lane];
+            }
+            gst(reinterpret_cast<uint4*>(pp + 16 * dt + 4 * j),
+                make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])));
+        }
+        if (j == 0) {
+            gst(pp + 64, M);
+            gst(pp + 65, L);
+        }
+    }
+}
+
 // ---- split merge + staging for the o projection ------------------------------------------
 // One wave per (sequence, head); lane = dim.  att = bf16(sum_s f_s o_s / sum_s f_s l_s),
 // f_s = exp(m_s - max m); written as the attention row and as the staged A words
@@ -399,6 +553,18 @@ hipError_t launch_rope_table(hipStream_t st, float* cs, int max_ctx, int half, f
 
 hipError_t launch_paged_attn(hipStream_t st, const PagedAttnArgs& a, int n_seq) {
     hipLaunchKernelGGL(paged_attn_kernel, dim3(a.max_splits, a.kvh, n_seq), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+// Rows of one sequence at consecutive positions up to last.
+hipError_t launch_prefill_attn(hipStream_t st, const PagedAttnArgs& a, int n, int last) {
+    const int tiles = (n + 15) / 16, splits = last / 256 + 1;
+    // the heads of a kv head share a workgroup's K and V unless that leaves CUs idle
+    int hper = a.grp;
+    while (hper > 1 && tiles * splits * a.kvh * ((a.grp + hper - 1) / hper) < 512) hper = (hper + 1) / 2;
+    const int hparts = (a.grp + hper - 1) / hper;
+    hipLaunchKernelGGL(prefill_attn_kernel, dim3(splits, a.kvh * hparts, tiles), dim3(256),
+                       16 * (hper * 8 + 1) * sizeof(uint4), st, a, n, hper);
     return hipGetLastError();
 }
 

@@ -95,6 +95,7 @@ hipError_t launch_stage(hipStream_t st, const uint16_t* x, int ldx, int M, int K
                         void* xs, float* xsum, uint16_t* hout, int32_t* pos_inc);
 hipError_t launch_embed_rows(hipStream_t st, const LinearDev& E, const int32_t* tokens, int n, uint16_t* x);
 hipError_t launch_rope_table(hipStream_t st, float* cs, int max_ctx, int half, float log2_theta);
+hipError_t launch_prefill_attn(hipStream_t st, const PagedAttnArgs& a, int n, int last);
 hipError_t launch_paged_attn(hipStream_t st, const PagedAttnArgs& a, int n_seq);
 hipError_t launch_merge_stage(hipStream_t st, const MergeArgs& a);
 // rows [n][pps] = n copies of table [pps]; pos [n] = p0, p0 + 1, ...

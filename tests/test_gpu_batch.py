@@ -437,3 +437,27 @@ def test_prefill_capacity_error(ming, ctx, small):
     with pytest.raises(ming.MingError) as e:
         b.prefill(pk, one_row_table(pk), 60, tokens=tok)  # 60 + 10 > 64
     assert e.value.status == ming.MING_E_CTX_OVER_CAPACITY
+
+
+@pytest.mark.parametrize("pos0,L", [(0, 64), (0, 300), (40, 65), (199, 79), (250, 512)])
+def test_prefill_row_tiles_equal_row_by_row(ming, ctx, small, pos0, L):
+    """The attention of 64 or more prompt rows (16-row tiles: ragged last tile, rows that end in different pages and
+    splits) against that of 32-row chunks (one row a workgroup), bit for bit."""
+    S, spec, syn, m, _, _ = small
+    pages = (pos0 + L + 63) // 64
+    x = ming.synth_normal_bf16(37, "prefill.tiles.x", L * spec.hidden).reshape(L, spec.hidden)
+    xd = torch.from_numpy(x.view(np.int16)).cuda().view(torch.bfloat16)
+    outs = []
+    for rows in (512, 32):
+        bt = ming.LmBatch(m, rows, 64 * pages)
+        pk = S.PagedKv(spec, 1, pages, spare=2, seed=7)
+        if pos0:
+            pk.fill_random([pos0], seed=38)
+        hid = torch.empty((L, spec.hidden), dtype=torch.bfloat16, device="cuda")
+        bt.prefill(pk, one_row_table(pk), pos0, x_in=xd, hidden=hid)
+        ctx.sync()
+        outs.append((hid, pk.gather(0, pos0 + L)))
+        bt.close()
+    (h0, (k0, v0)), (h1, (k1, v1)) = outs
+    assert torch.equal(h0, h1)
+    assert np.array_equal(k0, k1) and np.array_equal(v0, v1)
