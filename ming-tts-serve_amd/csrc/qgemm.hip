@@ -406,17 +406,18 @@ __device__ __forceinline__ void group_mma_pre(const AIn<MT>& in, const uint4 (&b
     }
 }
 
-template <int WM, int WN, int MT, int NW, int EPI>
+template <int WM, int WN, int MT, int NW, int GK, int EPI>
 __global__ __launch_bounds__(256) void qgemm_lds_kernel(QgemmArgs a, int kslices) {
     static_assert(WM * WN == 4, "four waves");
     constexpr int TPS = EPI == QE_SWIGLU ? NW / 2 : NW;
     constexpr int BM = 16 * WM * MT, NC = 16 * WN * NW;         // rows, weight columns of the tile
-    constexpr int AQ = BM * kLdsGK * 8 / 256;                   // activation uint4 per thread per chunk
-    static_assert(AQ * 256 == BM * kLdsGK * 8, "whole activation chunk per thread");
-    __shared__ uint4 As[2][BM * kRowStride];
-    __shared__ __align__(16) float Xs[2][kLdsGK * BM];          // group sums [group][row], read as float4
-    __shared__ uint4 Bs[2][NC * kRowStride];
-    __shared__ float2 Ss[2][NC * kLdsGK];                       // (scale, b - 128 scale)
+    constexpr int AQ = BM * GK * 8 / 256;                   // activation uint4 per thread per chunk
+    static_assert(AQ * 256 == BM * GK * 8 && NC * GK * 2 <= 256, "whole activation chunk, at most one weight quad per thread");
+    constexpr int RS = GK * 8 + 1;                              // uint4 per row / column in LDS (one of padding)
+    __shared__ uint4 As[2][BM * RS];
+    __shared__ __align__(16) float Xs[2][GK * BM];          // group sums [group][row], read as float4
+    __shared__ uint4 Bs[2][NC * RS];
+    __shared__ float2 Ss[2][NC * GK];                       // (scale, b - 128 scale)
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, c = lane % 16, j = lane / 16;
     const int wm = wave / WN, wn = wave % WN;
     int blk = blockIdx.x, si = 0;
@@ -438,71 +439,59 @@ __global__ __launch_bounds__(256) void qgemm_lds_kernel(QgemmArgs a, int kslices
         S = &pick(a, EPI == QE_SWIGLU ? (t < TPS ? 0 : 1) : si);
         return min(n0 + 16 * (wq * TPS + t % TPS) + k % 16, S->N - 1);
     };
-    // loads of a chunk: activations (AQ uint4 per thread), group sums (threads < kLdsGK BM / 4, one uint4),
-    // weights (threads < 2 kLdsGK NC: column k, group, half of 4 words), scales (threads < kLdsGK NC)
-    const int wk = tid / (2 * kLdsGK), wgg = (tid / 2) % kLdsGK, wh = tid % 2;
-    const bool wload = tid < NC * kLdsGK * 2;
+    // loads of a chunk: activations (AQ uint4 per thread), weights (column k, group, half of 4 words), group
+    // sums (one uint4 of 4 rows for the first GK BM / 4 threads) and scales (the first GK NC).  Every thread
+    // issues every load (the others repeat the last one's): a load that only some waves issue makes the wait
+    // for an older one wait for all.
+    const int wk = min(tid / (2 * GK), NC - 1), wgg = (tid / 2) % GK, wh = tid % 2;
+    const bool wload = tid < NC * GK * 2;
     const QSeg* WS;
-    const int wn_row = wcol(min(wk, NC - 1), WS);
+    const int wn_row = wcol(wk, WS);
     const uint32_t* wrow = WS->w + (size_t)wn_row * KW8;
-    const int sk = tid / kLdsGK, sgg = tid % kLdsGK;
-    const bool sload = tid < NC * kLdsGK;
+    const int sk = min(tid / GK, NC - 1), sgg = tid % GK;
+    const bool sload = tid < NC * GK, xload = tid < GK * BM / 4;
     const QSeg* SS;
-    const int sn = wcol(min(sk, NC - 1), SS);
-    const bool xload = tid < kLdsGK * BM / 4;
-    const int xgg = tid / (BM / 4), xr = (tid % (BM / 4)) * 4;  // group, first of 4 rows
+    const int sn = wcol(sk, SS);
+    const uint16_t *srow = SS->s + (size_t)sn * G, *brow = SS->b + (size_t)sn * G;
+    const int xt = min(tid, GK * BM / 4 - 1), xgg = xt / (BM / 4), xr = (xt % (BM / 4)) * 4;  // group, first of 4 rows
     const uint32_t mask = in_reg(0x000f000fu), magic = in_reg(kQ4Magic);
     const uint4* xs = static_cast<const uint4*>(a.xs);
-    const int nch = (G + kLdsGK - 1) / kLdsGK;
+    const int nch = (G + GK - 1) / GK;
     struct Raw {
         uint4 a[AQ], w, x;
-        uint32_t s, b;
+        uint16_t s, b;
     };
-    auto fetch = [&](int ch, Raw& R) {
+    auto fetch = [&](int ch, Raw& R) {  // groups past the last repeat it (their sums are not taken)
 #pragma unroll
-        for (int i = 0; i < AQ; i++) {  // uint4 q = tid + 256 i of the chunk: row q / (8 kLdsGK), group, word
-            const int q = tid + 256 * i, row = q / (8 * kLdsGK), gg = (q / 8) % kLdsGK, wd = q % 8;
-            const int g = min(ch * kLdsGK + gg, G - 1), m = min(r0 + row, Mp - 1);
+        for (int i = 0; i < AQ; i++) {  // uint4 q = tid + 256 i of the chunk: row q / (8 GK), group, word
+            const int q = tid + 256 * i, row = q / (8 * GK), gg = (q / 8) % GK, wd = q % 8;
+            const int g = min(ch * GK + gg, G - 1), m = min(r0 + row, Mp - 1);
             R.a[i] = ldg4(xs + ((size_t)g * Mp + m) * 8 + wd);
         }
-        if (xload) {
-            const int g = min(ch * kLdsGK + xgg, G - 1), m = min(r0 + xr, Mp - 4);
-            R.x = ldg4(a.xsum + (size_t)g * Mp + m);
-        }
-        const int g = ch * kLdsGK + wgg;
-        if (wload && g < G) R.w = ldg4(wrow + 8 * g + 4 * wh);
-        const int gs = ch * kLdsGK + sgg;
-        if (sload && gs < G) {
-            R.s = gld(SS->s + (size_t)sn * G + gs);
-            R.b = gld(SS->b + (size_t)sn * G + gs);
-        }
+        R.w = ldg4(wrow + 8 * min(ch * GK + wgg, G - 1) + 4 * wh);
+        R.x = ldg4(a.xsum + (size_t)min(ch * GK + xgg, G - 1) * Mp + min(r0 + xr, Mp - 4));
+        R.s = gld(srow + min(ch * GK + sgg, G - 1));
+        R.b = gld(brow + min(ch * GK + sgg, G - 1));
     };
     auto store = [&](const Raw& R, int buf) {
 #pragma unroll
         for (int i = 0; i < AQ; i++) {
-            const int q = tid + 256 * i, row = q / (8 * kLdsGK), gg = (q / 8) % kLdsGK, wd = q % 8;
-            As[buf][row * kRowStride + gg * 8 + wd] = R.a[i];
-        }
-        if (xload) {
-            Xs[buf][xgg * BM + xr] = __uint_as_float(R.x.x);
-            Xs[buf][xgg * BM + xr + 1] = __uint_as_float(R.x.y);
-            Xs[buf][xgg * BM + xr + 2] = __uint_as_float(R.x.z);
-            Xs[buf][xgg * BM + xr + 3] = __uint_as_float(R.x.w);
+            const int q = tid + 256 * i, row = q / (8 * GK), gg = (q / 8) % GK, wd = q % 8;
+            As[buf][row * RS + gg * 8 + wd] = R.a[i];
         }
         if (wload) {
             const uint32_t w4[4] = {R.w.x, R.w.y, R.w.z, R.w.w};
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const uint32_t w = w4[i];
-                Bs[buf][wk * kRowStride + wgg * 8 + 4 * wh + i] =
+                Bs[buf][wk * RS + wgg * 8 + 4 * wh + i] =
                     make_uint4((w & mask) | magic, ((w >> 4) & mask) | magic, ((w >> 8) & mask) | magic,
                                ((w >> 12) & mask) | magic);
             }
         }
-        if (sload) {
-            const float sv = bf2f((uint16_t)R.s), bv = bf2f((uint16_t)R.b);
-            Ss[buf][sk * kLdsGK + sgg] = make_float2(sv, fmaf(-128.0f, sv, bv));
-        }
+        if (xload) *reinterpret_cast<uint4*>(&Xs[buf][xgg * BM + xr]) = R.x;
+        const float sv = bf2f(R.s), bv = bf2f(R.b);
+        if (sload) Ss[buf][sk * GK + sgg] = make_float2(sv, fmaf(-128.0f, sv, bv));
     };
     f32x4_t acc[MT][NW], run[MT][NW];
 #pragma unroll
@@ -512,15 +501,15 @@ __global__ __launch_bounds__(256) void qgemm_lds_kernel(QgemmArgs a, int kslices
     const int gper = (G + kslices - 1) / kslices;
     auto chunk = [&](int ch, int buf) {
 #pragma unroll
-        for (int gg = 0; gg < kLdsGK; gg++) {
-            const int g = ch * kLdsGK + gg;
+        for (int gg = 0; gg < GK; gg++) {
+            const int g = ch * GK + gg;
             if (g >= G) break;
             AIn<MT> in;
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
                 const int row = 16 * (wm * MT + mt);
-                in.xa[mt][0] = As[buf][(row + c) * kRowStride + gg * 8 + 2 * j];
-                in.xa[mt][1] = As[buf][(row + c) * kRowStride + gg * 8 + 2 * j + 1];
+                in.xa[mt][0] = As[buf][(row + c) * RS + gg * 8 + 2 * j];
+                in.xa[mt][1] = As[buf][(row + c) * RS + gg * 8 + 2 * j + 1];
                 in.xsv[mt] = *reinterpret_cast<const float4*>(&Xs[buf][gg * BM + row + 4 * j]);
             }
             uint4 b[NW][2];
@@ -528,9 +517,9 @@ __global__ __launch_bounds__(256) void qgemm_lds_kernel(QgemmArgs a, int kslices
 #pragma unroll
             for (int t = 0; t < NW; t++) {
                 const int col = 16 * (wn * NW + t) + c;
-                b[t][0] = Bs[buf][col * kRowStride + gg * 8 + 2 * j];
-                b[t][1] = Bs[buf][col * kRowStride + gg * 8 + 2 * j + 1];
-                const float2 f = Ss[buf][col * kLdsGK + gg];
+                b[t][0] = Bs[buf][col * RS + gg * 8 + 2 * j];
+                b[t][1] = Bs[buf][col * RS + gg * 8 + 2 * j + 1];
+                const float2 f = Ss[buf][col * GK + gg];
                 sc[t] = f.x;
                 off[t] = f.y;
             }
@@ -546,23 +535,23 @@ __global__ __launch_bounds__(256) void qgemm_lds_kernel(QgemmArgs a, int kslices
             }
         }
     };
-    // two chunks' global loads in flight (register sets R0, R1) while one computes from LDS
-    Raw R0{}, R1{};
-    fetch(0, R0);
-    store(R0, 0);
-    if (nch > 1) fetch(1, R1);
-    if (nch > 2) fetch(2, R0);
-    __syncthreads();
-    for (int ch = 0; ch < nch; ch += 2) {
-        chunk(ch, 0);
-        if (ch + 1 < nch) store(R1, 1);
-        __syncthreads();
-        if (ch + 3 < nch) fetch(ch + 3, R1);
-        if (ch + 1 >= nch) break;
-        chunk(ch + 1, 1);
-        if (ch + 2 < nch) store(R0, 0);
-        __syncthreads();
-        if (ch + 4 < nch) fetch(ch + 4, R0);
+    // four chunks' global loads in flight in four register sets while one computes from LDS; the
+    // loads are issued past the last chunk too, so that the waits count the same on every path
+    Raw R[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) fetch(i, R[i]);
+    store(R[0], 0);
+    fetch(4, R[0]);
+    lds_sync();
+    for (int ch = 0;; ch += 4) {
+#define MING_LDS_STEP(I)                     \
+    chunk(ch + I, I % 2);                    \
+    if (ch + I + 1 >= nch) break;            \
+    store(R[(I + 1) % 4], (I + 1) % 2);      \
+    fetch(ch + I + 5, R[(I + 1) % 4]);       \
+    lds_sync();
+        MING_LDS_STEP(0) MING_LDS_STEP(1) MING_LDS_STEP(2) MING_LDS_STEP(3)
+#undef MING_LDS_STEP
     }
     // slices of the <= 64-row launch that hold no group add zero partials there
     for (int sidx = (G + gper - 1) / gper; sidx < kslices; sidx++)
@@ -689,13 +678,13 @@ __global__ __launch_bounds__(64 * WM * WN) void qgemm_wide_kernel(QgemmArgs a, i
         brow[i] = SS->b + (size_t)n * G;
     }
     const bool xload = tid < kLdsGK * BM / 4;
-    const int xgg = tid / (BM / 4), xr = (tid % (BM / 4)) * 4;
+    const int xt = min(tid, kLdsGK * BM / 4 - 1), xgg = xt / (BM / 4), xr = (xt % (BM / 4)) * 4;
     const uint32_t mask = in_reg(0x000f000fu), magic = in_reg(kQ4Magic);
     const uint4* xs = static_cast<const uint4*>(a.xs);
     const int nch = (G + kLdsGK - 1) / kLdsGK;
     struct Raw {
         uint4 a[AQ], w[WQ], x;
-        uint32_t s[SQ], b[SQ];
+        uint16_t s[SQ], b[SQ];
     };
     auto fetch = [&](int ch, Raw& R) {
 #pragma unroll
@@ -704,10 +693,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qgemm_wide_kernel(QgemmArgs a, i
             const int g = min(ch * kLdsGK + gg, G - 1), m = min(r0 + row, Mp - 1);
             R.a[i] = ldg4(xs + ((size_t)g * Mp + m) * 8 + wd);
         }
-        if (xload) {
-            const int g = min(ch * kLdsGK + xgg, G - 1), m = min(r0 + xr, Mp - 4);
-            R.x = ldg4(a.xsum + (size_t)g * Mp + m);
-        }
+        R.x = ldg4(a.xsum + (size_t)min(ch * kLdsGK + xgg, G - 1) * Mp + min(r0 + xr, Mp - 4));
 #pragma unroll
         for (int i = 0; i < WQ; i++) {
             const int q = tid + T * i, gg = (q / 2) % kLdsGK, wh = q % 2, g = min(ch * kLdsGK + gg, G - 1);
@@ -743,7 +729,7 @@ __global__ __launch_bounds__(64 * WM * WN) void qgemm_wide_kernel(QgemmArgs a, i
 #pragma unroll
         for (int i = 0; i < SQ; i++) {
             const int q = tid + T * i;
-            const float sv = bf2f((uint16_t)R.s[i]), bv = bf2f((uint16_t)R.b[i]);
+            const float sv = bf2f(R.s[i]), bv = bf2f(R.b[i]);
             Ss[buf][q] = make_float2(sv, fmaf(-128.0f, sv, bv));  // q = column * kLdsGK + group
         }
     };
@@ -789,22 +775,24 @@ __global__ __launch_bounds__(64 * WM * WN) void qgemm_wide_kernel(QgemmArgs a, i
             }
         }
     };
-    Raw R0{}, R1{};
-    fetch(0, R0);
-    store(R0, 0);
-    if (nch > 1) fetch(1, R1);
-    if (nch > 2) fetch(2, R0);
-    __syncthreads();
-    for (int ch = 0; ch < nch; ch += 2) {
+    // two chunks' loads in flight, issued past the last chunk too (as qgemm_lds_kernel)
+    Raw R[2];
+    fetch(0, R[0]);
+    fetch(1, R[1]);
+    store(R[0], 0);
+    fetch(2, R[0]);
+    lds_sync();
+    for (int ch = 0;; ch += 2) {
         chunk(ch, 0);
-        if (ch + 1 < nch) store(R1, 1);
-        __syncthreads();
-        if (ch + 3 < nch) fetch(ch + 3, R1);
         if (ch + 1 >= nch) break;
+        store(R[1], 1);
+        fetch(ch + 3, R[1]);
+        lds_sync();
         chunk(ch + 1, 1);
-        if (ch + 2 < nch) store(R0, 0);
-        __syncthreads();
-        if (ch + 4 < nch) fetch(ch + 4, R0);
+        if (ch + 2 >= nch) break;
+        store(R[0], 0);
+        fetch(ch + 4, R[0]);
+        lds_sync();
     }
     for (int sidx = (G + gper - 1) / gper; sidx < kslices; sidx++)
 #pragma unroll
@@ -1174,7 +1162,7 @@ hipError_t launch_mt(hipStream_t st, const QgemmArgs& a) {
 
 // More than 64 rows: qgemm_lds_kernel with the K slices of the shape's launch for
 // <= 64 rows (GPW, KWMAX as there); WM x WN waves of MT x NW tiles.
-template <int WM, int WN, int MT, int NW, int GPW, int KWMAX, int EPI>
+template <int WM, int WN, int MT, int NW, int GK, int GPW, int KWMAX, int EPI>
 hipError_t launch_big(hipStream_t st, QgemmArgs a) {
     constexpr int TPS = EPI == QE_SWIGLU ? NW / 2 : NW, CB = 16 * TPS * WN, BM = 16 * WM * MT;
     const int G = a.K / 64, kw = GPW == 0 ? KWMAX : min(KWMAX, (G + GPW - 1) / GPW);
@@ -1184,7 +1172,7 @@ hipError_t launch_big(hipStream_t st, QgemmArgs a) {
         if (EPI != QE_SWIGLU && a.nseg > 1 && a.seg[i].N % CB) return hipErrorInvalidValue;
     const int grid = a.blocks[0] + a.blocks[1] + a.blocks[2];
     const int mtt = (a.M + 15) / 16, gy = (16 * mtt + BM - 1) / BM;
-    hipLaunchKernelGGL((qgemm_lds_kernel<WM, WN, MT, NW, EPI>), dim3(grid, gy), dim3(256), 0, st, a, kw);
+    hipLaunchKernelGGL((qgemm_lds_kernel<WM, WN, MT, NW, GK, EPI>), dim3(grid, gy), dim3(256), 0, st, a, kw);
     return hipGetLastError();
 }
 
@@ -1227,6 +1215,9 @@ bool launch_wide(hipStream_t st, QgemmArgs a, hipError_t& err) {
 // whose 32 x 32 tiles (one 16 x 16 tile per wave) give a 512-row chunk 448
 // workgroups at N = 896 instead of 112 (512-token prefill 3.58 -> 3.20 ms;
 // 64 x 32, 32 x 64, 64 x 16 and 16 x 64 tiles measured 3.24-3.35 ms).
+// The residual projections take K from 2048 in LDS chunks of four groups (half the barriers:
+// K = 4864, N = 896, 65 .. 256 rows 29.0 -> 23.6 us, 512 rows 33.9 -> 32.8) and shorter ones in
+// chunks of two (K = 896, 512 rows: 9.3 us, 9.8 with four).
 hipError_t launch_qgemm_epi(hipStream_t st, QgemmArgs a, int epi) {
     if (a.M < 1 || a.M > kQgemmMaxRows || a.K % 64 || a.nseg < 1 || a.nseg > 3) return hipErrorInvalidValue;
     const bool big = a.M > 64;
@@ -1243,10 +1234,11 @@ hipError_t launch_qgemm_epi(hipStream_t st, QgemmArgs a, int epi) {
             }
             if (a.pmax) return hipErrorInvalidValue;
             set_blocks(16);
-            return big ? launch_big<2, 2, 2, 2, 5, 16, QE_PLAIN>(st, a) : launch_mt<1, 5, 16, QE_PLAIN, 1>(st, a);
+            return big ? launch_big<2, 2, 2, 2, 2, 5, 16, QE_PLAIN>(st, a) : launch_mt<1, 5, 16, QE_PLAIN, 1>(st, a);
         case QE_RES:
             set_blocks(16);
-            return big ? launch_big<2, 2, 1, 1, 5, 16, QE_RES>(st, a) : launch_mt<1, 5, 16, QE_RES, 1>(st, a);
+            if (!big) return launch_mt<1, 5, 16, QE_RES, 1>(st, a);
+            return a.K >= 2048 ? launch_big<2, 2, 1, 1, 4, 5, 16, QE_RES>(st, a) : launch_big<2, 2, 1, 1, 2, 5, 16, QE_RES>(st, a);
         case QE_SWIGLU:
             if (a.nseg != 2 || a.seg[0].N != a.seg[1].N) return hipErrorInvalidValue;
             set_blocks(32);
@@ -1254,7 +1246,7 @@ hipError_t launch_qgemm_epi(hipStream_t st, QgemmArgs a, int epi) {
             if (big) {
                 hipError_t e;
                 if (launch_wide<2, 4, 2, 4, 0, 2, QE_SWIGLU>(st, a, e)) return e;
-                return launch_big<2, 2, 2, 2, 0, 2, QE_SWIGLU>(st, a);
+                return launch_big<2, 2, 2, 2, 2, 0, 2, QE_SWIGLU>(st, a);
             }
             return launch_mt<4, 0, 2, QE_SWIGLU, 2>(st, a);
         case QE_QKV:
@@ -1262,7 +1254,7 @@ hipError_t launch_qgemm_epi(hipStream_t st, QgemmArgs a, int epi) {
             for (int i = 0; i < 3; i++)
                 if (a.seg[i].N % 64) return hipErrorInvalidValue;
             set_blocks(64);
-            return big ? launch_big<4, 1, 1, 4, 2, 8, QE_QKV>(st, a) : launch_mt<4, 2, 8, QE_QKV, 1>(st, a);
+            return big ? launch_big<4, 1, 1, 4, 2, 2, 8, QE_QKV>(st, a) : launch_mt<4, 2, 8, QE_QKV, 1>(st, a);
         default:
             return hipErrorInvalidValue;
     }
