@@ -233,19 +233,32 @@ constexpr int kSmallNT = EPI == VE_SWIGLU ? 4 : (EPI == VE_QKV ? 2 : 1);
 template <int EPI>
 constexpr int kSmallWaves = kSmallNT<EPI> == 1 ? 10 : 8;
 
+// The weights of a chunk come by quads of lanes (lane l: 16 bytes of row l / 4; bf16: the 64
+// bytes of a 32-k step, 4-bit: the 64 bytes of two groups) and each wave turns them round in LDS
+// of its own: a load of 16 rows in the operand's order (16 consecutive lanes on 16 rows) takes the
+// address unit four times as long, and a 4-bit group took four of them a tile (two words, scale,
+// bias), more than all the activations.  The scales and biases of two groups are one load: lane
+// 16 x + c the value x of column c, (s, s', b, b').
+constexpr int kQRow = 20;  // dwords of a 4-bit row's two groups in LDS (16, padded: no bank conflicts)
+template <int WF, int MT, int NT>
+constexpr int kSmallLds() {  // bytes a wave: its turned weights, and after the loop its sums
+    const int turn = WF == VW_Q4 ? NT * (16 * kQRow + 64) * 4 : 2 * NT * 1024, sums = MT * NT * 1024;
+    return turn > sums ? turn : sums;
+}
+
 template <int WF, int NP, int MT, int NT>
-struct V3Unit {
-    uint4 a[kUnitK<WF> / 32][NP][MT];
-    uint4 w[WF == VW_Q4 ? 1 : NT];
-    uint32_t q[WF == VW_Q4 ? NT : 1][2];
-    uint16_t s[NT], b[NT];
+struct V3Chunk {
+    uint4 a[kSmallCh<WF>][kUnitK<WF> / 32][NP][MT];
+    uint4 w[WF == VW_Q4 ? 1 : kSmallCh<WF>][NT];
+    uint16_t sb[NT];
 };
 
 template <int WF, int EPI, int NP, int MT>
 __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g) {
     constexpr int NT = kSmallNT<EPI>;
     constexpr int UK = kUnitK<WF>, UH = UK / 32, CH = kSmallCh<WF>;
-    extern __shared__ float red[];  // [waves][MT * 4][NT][64]
+    extern __shared__ __align__(16) float vs_lds[];  // [waves][kSmallLds]
+    constexpr int LW = kSmallLds<WF, MT, NT>() / 4;
     const int W = blockDim.x / kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave, c = lane % 16, j = lane / 16;
     const int m0 = blockIdx.y * 16 * MT, z = blockIdx.z;
@@ -255,7 +268,7 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
     for (int t = 0; t < NT; t++) col[t] = c0 + (EPI == VE_QKV ? 32 * t : 16 * (t % 2)) + c;
     const V3View<WF, EPI> v = load_view<WF, EPI>(g, c0);
     const int U = v.K / UK, per = (U + v.ks - 1) / v.ks, u0 = z * per, u1 = min(U, u0 + per);
-    // 32-bit byte offsets per lane from uniform bases (operands: row tile; weights: row)
+    // 32-bit byte offsets per lane from uniform bases (operands: row tile; weights: row lane / 4)
     uint32_t ao[MT], wo[NT], so[NT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
@@ -263,9 +276,8 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
                          : (uint32_t)min(m0 / 16 + mt, (v.M - 1) / 16) * (v.K / 32) * 1024u + 16u * lane;
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        const uint32_t n = min(col[t] - v.start, v.n - 1);
-        wo[t] = WF == VW_Q4 ? n * (v.K / 2) + 4u * j : n * v.K * 2u + 16u * j;
-        so[t] = n * (v.K / 64) * 2u;
+        wo[t] = (uint32_t)min(col[t] - c - v.start + lane / 4, v.n - 1) * (WF == VW_Q4 ? v.K / 2 : v.K * 2) + 16u * (lane % 4);
+        so[t] = (uint32_t)min(col[t] - v.start, v.n - 1) * (v.K / 64) * 2u;
     }
     auto at = [](const void* base, uint32_t off) { return static_cast<const char*>(base) + off; };
     f32x4_t hi[MT][NT], lo[MT][NT];
@@ -273,91 +285,120 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int t = 0; t < NT; t++) hi[mt][t] = lo[mt][t] = kZero4;
-    auto load = [&](int u, V3Unit<WF, NP, MT, NT>& in) {
+    float* mine = vs_lds + wave * LW;
+    auto load = [&](int u, V3Chunk<WF, NP, MT, NT>& in) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const bool up = EPI == VE_SWIGLU && t >= NT / 2;
             const char* w = up ? v.wu : v.w;
             if (WF == VW_Q4) {
-#pragma unroll
-                for (int h = 0; h < 2; h++)
-                    in.q[t][h] = gld(reinterpret_cast<const uint32_t*>(at(w + 32 * (size_t)u + 16 * h, wo[t])));
-                in.s[t] = gld(reinterpret_cast<const uint16_t*>(at((up ? v.su : v.s) + u, so[t])));
-                in.b[t] = gld(reinterpret_cast<const uint16_t*>(at((up ? v.bu : v.b) + u, so[t])));
+                const bool two = u + 1 < u1;  // a last single group is read twice
+                in.w[0][t] = ldg4(at(w + 32 * (size_t)u, wo[t] - (!two && lane % 4 >= 2 ? 32u : 0u)));
+                const uint16_t* sv = up ? v.su : v.s;
+                const uint16_t* bv = up ? v.bu : v.b;
+                const char* p = at(j < 2 ? sv : bv, so[t]);
+                in.sb[t] = gld(reinterpret_cast<const uint16_t*>(p) + u + (two ? j % 2 : 0));
             } else {
-                in.w[t] = ldg4(at(w + 64 * (size_t)u, wo[t]));
+#pragma unroll
+                for (int k = 0; k < CH; k++)
+                    if (u + k < u1) in.w[k][t] = ldg4(at(w + 64 * (size_t)(u + k), wo[t]));
             }
         }
 #pragma unroll
-        for (int h = 0; h < UH; h++)
+        for (int k = 0; k < CH; k++)
+            if (u + k < u1)
 #pragma unroll
-            for (int p = 0; p < NP; p++)
+                for (int h = 0; h < UH; h++)
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                    in.a[h][p][mt] = ldg4(at(v.a + p * v.aps + ((size_t)u * UH + h) * (NP == 1 ? 32 : 512), ao[mt]));
+                    for (int p = 0; p < NP; p++)
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++)
+                            in.a[k][h][p][mt] =
+                                ldg4(at(v.a + p * v.aps + ((size_t)(u + k) * UH + h) * (NP == 1 ? 32 : 512), ao[mt]));
     };
     const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
     const uint32_t mask = in_reg(kQ16Mask), magic = in_reg(kQ16Magic);
-    auto work = [&](const V3Unit<WF, NP, MT, NT>& in) {
+    auto work = [&](const V3Chunk<WF, NP, MT, NT>& in, int n) {  // n units
         if constexpr (WF == VW_Q4) {
-            // the group sums of x, in every column's place
-            f32x4_t xs[MT];
-            uint4 x[2][NP][MT];
-#pragma unroll
-            for (int h = 0; h < 2; h++)
-#pragma unroll
-                for (int p = 0; p < NP; p++)
-#pragma unroll
-                    for (int mt = 0; mt < MT; mt++) x[h][p][mt] = NP == 1 ? pair_order(in.a[h][p][mt]) : in.a[h][p][mt];
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                xs[mt] = kZero4;
-#pragma unroll
-                for (int p = NP - 1; p >= 0; p--) xs[mt] = mma(x[1][p][mt], ones, mma(x[0][p][mt], ones, xs[mt]));
-            }
+            uint32_t* q = reinterpret_cast<uint32_t*>(mine);  // [tile][16 rows][kQRow], [tile][s, s', b, b'][16]
+            uint32_t* sc = q + NT * 16 * kQRow;
 #pragma unroll
             for (int t = 0; t < NT; t++) {
-                const uint4 b0 = unpack_q16(in.q[t][0], mask, magic), b1 = unpack_q16(in.q[t][1], mask, magic);
-                const float s = bf2f(in.s[t]), off = fmaf(-16.0f, s, bf2f(in.b[t]));
+                *reinterpret_cast<uint4*>(q + (16 * t + lane / 4) * kQRow + 4 * (lane % 4)) = in.w[0][t];
+                sc[64 * t + lane] = (uint32_t)in.sb[t] << 16;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the reads below are of other types and lanes
+#pragma unroll
+            for (int k = 0; k < CH; k++) {
+                if (k >= n) break;
+                // the group sums of x, in every column's place
+                f32x4_t xs[MT];
+                uint4 x[2][NP][MT];
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int p = 0; p < NP; p++)
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++)
+                            x[h][p][mt] = NP == 1 ? pair_order(in.a[k][h][p][mt]) : in.a[k][h][p][mt];
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) {
-                    f32x4_t h = kZero4;
+                    xs[mt] = kZero4;
 #pragma unroll
-                    for (int p = NP - 1; p >= 0; p--) h = mma(x[1][p][mt], b1, mma(x[0][p][mt], b0, h));
+                    for (int p = NP - 1; p >= 0; p--) xs[mt] = mma(x[1][p][mt], ones, mma(x[0][p][mt], ones, xs[mt]));
+                }
 #pragma unroll
-                    for (int r = 0; r < 4; r++) hi[mt][t][r] = fmaf(s, h[r], fmaf(off, xs[mt][r], hi[mt][t][r]));
+                for (int t = 0; t < NT; t++) {
+                    const uint32_t* qr = q + (16 * t + c) * kQRow + 8 * k + j;
+                    const uint4 b0 = unpack_q16(qr[0], mask, magic), b1 = unpack_q16(qr[4], mask, magic);
+                    const float s = __uint_as_float(sc[64 * t + 16 * k + c]),
+                                off = fmaf(-16.0f, s, __uint_as_float(sc[64 * t + 32 + 16 * k + c]));
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) {
+                        f32x4_t h = kZero4;
+#pragma unroll
+                        for (int p = NP - 1; p >= 0; p--) h = mma(x[1][p][mt], b1, mma(x[0][p][mt], b0, h));
+#pragma unroll
+                        for (int r = 0; r < 4; r++) hi[mt][t][r] = fmaf(s, h[r], fmaf(off, xs[mt][r], hi[mt][t][r]));
+                    }
                 }
             }
         } else {
+            // 16 rows of 4 blocks of 16 bytes, the block permuted by the row: no bank conflicts either way
+            uint4* wt = reinterpret_cast<uint4*>(mine);
 #pragma unroll
-            for (int p = 0; p < NP; p++)
+            for (int k = 0; k < CH; k++) {
+                if (k >= n) break;
+                uint4 w[NT];
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
+                for (int t = 0; t < NT; t++) wt[(k % 2 * NT + t) * 64 + 4 * (lane / 4) + (lane % 4 ^ lane / 16)] = in.w[k][t];
 #pragma unroll
-                    for (int t = 0; t < NT; t++) {
-                        f32x4_t& acc = p == 0 ? hi[mt][t] : lo[mt][t];
-                        acc = mma(in.a[0][p][mt], in.w[t], acc);
-                    }
+                for (int t = 0; t < NT; t++) w[t] = wt[(k % 2 * NT + t) * 64 + 4 * c + (j ^ c / 4)];
+#pragma unroll
+                for (int p = 0; p < NP; p++)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                        for (int t = 0; t < NT; t++) {
+                            f32x4_t& acc = p == 0 ? hi[mt][t] : lo[mt][t];
+                            acc = mma(in.a[k][0][p][mt], w[t], acc);
+                        }
+            }
         }
     };
     for (int ub = u0 + wave * CH; ub < u1; ub += W * CH) {
         // a fresh scalar each time round: the loads keep their uniform base + lane offset form
         const int u = __builtin_amdgcn_readfirstlane(ub);
-        V3Unit<WF, NP, MT, NT> in[CH];
-#pragma unroll
-        for (int k = 0; k < CH; k++)
-            if (u + k < u1) load(u + k, in[k]);
-#pragma unroll
-        for (int k = 0; k < CH; k++)
-            if (u + k < u1) work(in[k]);
+        V3Chunk<WF, NP, MT, NT> in;
+        load(u, in);
+        work(in, u1 - u);
     }
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int t = 0; t < NT; t++)
-                red[(((wave * MT + mt) * 4 + r) * NT + t) * kWave + lane] = hi[mt][t][r] + lo[mt][t][r];
+            for (int t = 0; t < NT; t++) mine[((mt * 4 + r) * NT + t) * kWave + lane] = hi[mt][t][r] + lo[mt][t][r];
     __syncthreads();
     for (int u = wave; u < MT * 4; u += W) {  // row slot u = 4 mt + r
         const int row = m0 + 16 * (u / 4) + 4 * j + u % 4;
@@ -365,8 +406,8 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
         float x[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            float s = red[(u * NT + t) * kWave + lane];
-            for (int w = 1; w < W; w++) s += red[((w * MT * 4 + u) * NT + t) * kWave + lane];
+            float s = vs_lds[(u * NT + t) * kWave + lane];
+            for (int w = 1; w < W; w++) s += vs_lds[w * LW + (u * NT + t) * kWave + lane];
             x[t] = s;
         }
         v3_epi<WF, EPI, NT>(v, row, col, x, z);
@@ -733,11 +774,10 @@ hipError_t launch_small(hipStream_t st, const V3Gemm& g, int N) {
     // twice the CUs pull the activations
     const int mt = g.M > 16 && gx * g.ks >= kSmallTwoTiles ? 2 : 1;
     const dim3 grid(gx, (g.M + 16 * mt - 1) / (16 * mt), g.ks);
-    const size_t lds = sizeof(float) * (size_t)W * mt * 4 * NT * kWave;
     if (mt == 2)
-        hipLaunchKernelGGL((vsmall_kernel<WF, EPI, NP, 2>), grid, dim3(64 * W), lds, st, g);
+        hipLaunchKernelGGL((vsmall_kernel<WF, EPI, NP, 2>), grid, dim3(64 * W), (size_t)W * (kSmallLds<WF, 2, NT>()), st, g);
     else
-        hipLaunchKernelGGL((vsmall_kernel<WF, EPI, NP, 1>), grid, dim3(64 * W), lds, st, g);
+        hipLaunchKernelGGL((vsmall_kernel<WF, EPI, NP, 1>), grid, dim3(64 * W), (size_t)W * (kSmallLds<WF, 1, NT>()), st, g);
     return hipGetLastError();
 }
 
