@@ -70,14 +70,34 @@ struct GroupIn {
     float4 xsv[MT];     // group sums of rows 16 mt + 4j + r, r = 0..3
 };
 
+// Two groups' loads of one lane.  A load in the operand's order puts 16 consecutive lanes on 16
+// rows, and the address unit takes such a load lane by lane (four times as long as lanes on
+// consecutive 16 bytes); a group had five to eight of them a tile, which bound these kernels.  So
+// the two groups' packed words come by quads (lane l: 16 bytes of weight row l / 4), the staged
+// activations as they lie (1 KB a load) and scales and biases in one load (lane 16 x + c: value x
+// of column c in (s, s', b, b')), and the wave turns them round in LDS of its own: 13 rows, N = 896,
+// K = 4864 10.4 -> 6.3 us, gate/up 8.1 -> 7.3; 64 rows 10.9 -> 6.7 and 13.4 -> 11.9.
+template <int MT, int NW>
+struct PairIn {
+    uint4 w[NW], xa[2][MT][2];
+    float4 xsv[2][MT];
+    uint16_t sb[NW];
+};
+constexpr int kQRow = 20;  // dwords of a weight row's two groups in LDS (16, padded against bank conflicts)
+template <int MT, int NW>
+constexpr int wave_lds() {  // bytes a wave: weights, scales, one group's activations; after the loop its sums
+    const int turn = NW * (16 * kQRow + 64) * 4 + MT * 2048, sums = MT * NW * 1024;
+    return turn > sums ? turn : sums;
+}
+
 // Per-lane 32-bit byte offsets from the uniform bases: the loads then take a
 // scalar base plus a 32-bit vector offset, with no per-load 64-bit arithmetic.
-template <int MT, int NW>
+template <int NW>
 struct Offs {
-    uint32_t w[NW];     // row n_t * K/2 + 8j
-    uint32_t s[NW];     // row n_t * G * 2
-    uint32_t x;         // ((16 mt0 + c) * 8 + 2j) * 16     (+ g * Mp * 128 + 2048 mt)
-    uint32_t xs;        // (16 mt0 + 4j) * 4                  (+ g * Mp * 4 + 64 mt)
+    uint32_t w[NW];     // row n(l / 4) * K/2 + 16 (l % 4)
+    uint32_t s[NW];     // row n(c) * G * 2
+    uint32_t x;         // 16 mt0 * 128 + 16 l            (+ g * Mp * 128 + 2048 mt + 1024 h)
+    uint32_t xs;        // (16 mt0 + 4j) * 4              (+ g * Mp * 4 + 64 mt)
 };
 
 template <class T>
@@ -85,24 +105,29 @@ __device__ __forceinline__ const T* at(const T* base, uint32_t byte_off) {
     return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + byte_off);
 }
 
+// Groups g and g + 1 (two: the slice holds both; else the first one's are read again).
 template <int MT, int NW>
-__device__ __forceinline__ void group_load(const QgemmArgs& a, const uint32_t* const (&wb)[NW],
-                                           const uint16_t* const (&sb)[NW], const uint16_t* const (&bb)[NW],
-                                           const Offs<MT, NW>& o, int Mp, int g, GroupIn<MT, NW>& in) {
+__device__ __forceinline__ void pair_load(const QgemmArgs& a, const uint32_t* const (&wb)[NW],
+                                          const uint16_t* const (&sb)[NW], const uint16_t* const (&bb)[NW],
+                                          const Offs<NW>& o, int Mp, int g, bool two, PairIn<MT, NW>& in) {
+    const int lane = threadIdx.x % kWave, j = lane / 16;
     const uint4* xs = static_cast<const uint4*>(a.xs);
+    const uint32_t back = !two && lane % 4 >= 2 ? 32u : 0u, g1 = two ? 1 : 0;
 #pragma unroll
     for (int t = 0; t < NW; t++) {
-        in.wq[t] = ldg2(at(wb[t], o.w[t] + 32u * g));
-        in.sc[t] = bf2f(gld(at(sb[t], o.s[t] + 2u * g)));
-        in.bi[t] = bf2f(gld(at(bb[t], o.s[t] + 2u * g)));
+        in.w[t] = ldg4(at(wb[t], o.w[t] + 32u * g - back));
+        in.sb[t] = gld(at(j < 2 ? sb[t] : bb[t], o.s[t] + 2u * (g + (j % 2) * g1)));
     }
-    const uint32_t xg = o.x + (uint32_t)g * Mp * 128u, sg = o.xs + (uint32_t)g * Mp * 4u;
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        in.xa[mt][0] = ldg4(at(xs, xg + 2048u * mt));
-        in.xa[mt][1] = ldg4(at(xs, xg + 2048u * mt + 16u));
-        const uint4 v = ldg4(at(a.xsum, sg + 64u * mt));
-        in.xsv[mt] = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+    for (int k = 0; k < 2; k++) {
+        const uint32_t gk = g + (k ? g1 : 0), xg = o.x + gk * Mp * 128u, sg = o.xs + gk * Mp * 4u;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            in.xa[k][mt][0] = ldg4(at(xs, xg + 2048u * mt));
+            in.xa[k][mt][1] = ldg4(at(xs, xg + 2048u * mt + 1024u));
+            const uint4 v = ldg4(at(a.xsum, sg + 64u * mt));
+            in.xsv[k][mt] = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+        }
     }
 }
 
@@ -136,6 +161,47 @@ __device__ __forceinline__ void group_mma(const GroupIn<MT, NW>& in, f32x4_t (&a
     for (int t = 0; t < NW; t++) {
         if (t + 1 < NW) issue(t + 1, ag[(t + 1) & 1]);
         fold(t, ag[t & 1]);
+    }
+}
+
+// The n (1 or 2) groups of a pair through the wave's LDS (lds: wave_lds bytes) and into acc.
+template <int MT, int NW>
+__device__ __forceinline__ void pair_mma(const PairIn<MT, NW>& p, int n, uint32_t* lds, f32x4_t (&acc)[MT][NW],
+                                         uint32_t mask, uint32_t magic) {
+    const int lane = threadIdx.x % kWave, c = lane % 16, j = lane / 16;
+    uint32_t *q = lds, *sc = q + NW * 16 * kQRow;
+    uint4* xl = reinterpret_cast<uint4*>(sc + NW * 64);  // [MT][16 rows][8 words], words permuted by the row
+#pragma unroll
+    for (int t = 0; t < NW; t++) {
+        *reinterpret_cast<uint4*>(q + (16 * t + lane / 4) * kQRow + 4 * (lane % 4)) = p.w[t];
+        sc[64 * t + lane] = (uint32_t)p.sb[t] << 16;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        if (k >= n) break;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int row = 8 * h + lane / 8;
+                xl[128 * mt + 8 * row + (lane % 8 ^ row / 2)] = p.xa[k][mt][h];
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes' and types' values are read below
+        GroupIn<MT, NW> in;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            in.xa[mt][0] = xl[128 * mt + 8 * c + (2 * j ^ c / 2)];
+            in.xa[mt][1] = xl[128 * mt + 8 * c + ((2 * j + 1) ^ c / 2)];
+            in.xsv[mt] = p.xsv[k][mt];
+        }
+#pragma unroll
+        for (int t = 0; t < NW; t++) {
+            const uint32_t* w = q + (16 * t + c) * kQRow + 8 * k + 2 * j;
+            in.wq[t] = make_uint2(w[0], w[1]);
+            in.sc[t] = __uint_as_float(sc[64 * t + 16 * k + c]);
+            in.bi[t] = __uint_as_float(sc[64 * t + 32 + 16 * k + c]);
+        }
+        group_mma<MT, NW>(in, acc, mask, magic);
     }
 }
 
@@ -247,12 +313,12 @@ __device__ __forceinline__ void epi_row(const QgemmArgs& a, const QSeg& S, int s
     }
 }
 
-// KW = blockDim.x / 64 waves (<= KWMAX) split the K/64 groups; each wave takes
-// its groups either through a three-deep register ring (GPW = 0) or in chunks
-// of GPW whose loads are all issued before the chunk's MFMAs.
-template <int MT, int NW, int GPW, int KWMAX, int EPI>
+// KW = blockDim.x / 64 waves (<= KWMAX) split the K/64 groups; each wave takes its groups two at a
+// time, the next two pairs' loads in flight.
+template <int MT, int NW, int KWMAX, int EPI>
 __global__ __launch_bounds__(64 * KWMAX) void qgemm_kernel(QgemmArgs a) {
-    extern __shared__ float red[];  // [KW][MT * 4][NW][64]
+    extern __shared__ __align__(16) float red[];  // [KW][wave_lds]
+    constexpr int LW = wave_lds<MT, NW>() / 4;
     constexpr int TPS = EPI == QE_SWIGLU ? NW / 2 : NW;  // column tiles per segment and workgroup
     const int KW = blockDim.x / kWave;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, c = lane % 16, j = lane / 16;
@@ -271,18 +337,18 @@ __global__ __launch_bounds__(64 * KWMAX) void qgemm_kernel(QgemmArgs a) {
     const uint32_t* wb[NW];
     const uint16_t* sb[NW];
     const uint16_t* bb[NW];
-    Offs<MT, NW> o;
+    Offs<NW> o;
 #pragma unroll
     for (int t = 0; t < NW; t++) {
         const QSeg& S = pick(a, EPI == QE_SWIGLU ? (t < TPS ? 0 : 1) : si);
-        const int n = min(n0 + 16 * (t % TPS) + c, S.N - 1);
+        const int n = n0 + 16 * (t % TPS);
         wb[t] = S.w;
         sb[t] = S.s;
         bb[t] = S.b;
-        o.w[t] = (uint32_t)n * KW8 * 4u + 8u * j;
-        o.s[t] = (uint32_t)n * G * 2u;
+        o.w[t] = (uint32_t)min(n + lane / 4, S.N - 1) * KW8 * 4u + 16u * (lane % 4);
+        o.s[t] = (uint32_t)min(n + c, S.N - 1) * G * 2u;
     }
-    o.x = ((uint32_t)(16 * mt0 + c) * 8u + 2u * j) * 16u;
+    o.x = (uint32_t)(16 * mt0) * 128u + 16u * lane;
     o.xs = (uint32_t)(16 * mt0 + 4 * j) * 4u;
     const int gper = (G + KW - 1) / KW, g0 = wave * gper, g1 = min(G, g0 + gper);
     f32x4_t acc[MT][NW];
@@ -291,33 +357,17 @@ __global__ __launch_bounds__(64 * KWMAX) void qgemm_kernel(QgemmArgs a) {
 #pragma unroll
         for (int t = 0; t < NW; t++) acc[mt][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t mask = in_reg(0x000f000fu), magic = in_reg(kQ4Magic);
-    if constexpr (GPW == 0) {
-        // a ring of three groups in registers: two groups' loads in flight while one computes
-        if (g0 < g1) {
-            GroupIn<MT, NW> b0, b1, b2;
-            group_load<MT, NW>(a, wb, sb, bb, o, Mp, g0, b0);
-            if (g0 + 1 < g1) group_load<MT, NW>(a, wb, sb, bb, o, Mp, g0 + 1, b1);
-            for (int g = g0; g < g1; g += 3) {
-                if (g + 2 < g1) group_load<MT, NW>(a, wb, sb, bb, o, Mp, g + 2, b2);
-                group_mma<MT, NW>(b0, acc, mask, magic);
-                if (g + 1 >= g1) break;
-                if (g + 3 < g1) group_load<MT, NW>(a, wb, sb, bb, o, Mp, g + 3, b0);
-                group_mma<MT, NW>(b1, acc, mask, magic);
-                if (g + 2 >= g1) break;
-                if (g + 4 < g1) group_load<MT, NW>(a, wb, sb, bb, o, Mp, g + 4, b1);
-                group_mma<MT, NW>(b2, acc, mask, magic);
-            }
-        }
-    } else {
-        // chunks of GPW groups whose loads are all issued before the chunk's MFMAs
-        for (int gb = g0; gb < g1; gb += GPW) {
-            GroupIn<MT, NW> in[GPW];
-#pragma unroll
-            for (int u = 0; u < GPW; u++)
-                if (gb + u < g1) group_load<MT, NW>(a, wb, sb, bb, o, Mp, gb + u, in[u]);
-#pragma unroll
-            for (int u = 0; u < GPW; u++)
-                if (gb + u < g1) group_mma<MT, NW>(in[u], acc, mask, magic);
+    uint32_t* mine = reinterpret_cast<uint32_t*>(red + wave * LW);
+    if (g0 < g1) {
+        PairIn<MT, NW> p0, p1;
+        pair_load<MT, NW>(a, wb, sb, bb, o, Mp, g0, g0 + 1 < g1, p0);
+        if (g0 + 2 < g1) pair_load<MT, NW>(a, wb, sb, bb, o, Mp, g0 + 2, g0 + 3 < g1, p1);
+        for (int g = g0; g < g1; g += 4) {
+            pair_mma<MT, NW>(p0, g1 - g, mine, acc, mask, magic);
+            if (g + 4 < g1) pair_load<MT, NW>(a, wb, sb, bb, o, Mp, g + 4, g + 5 < g1, p0);
+            if (g + 2 >= g1) break;
+            pair_mma<MT, NW>(p1, g1 - g - 2, mine, acc, mask, magic);
+            if (g + 6 < g1) pair_load<MT, NW>(a, wb, sb, bb, o, Mp, g + 6, g + 7 < g1, p1);
         }
     }
     // the waves' partial sums through LDS; wave w then owns the row slots u = mt * 4 + r with u % KW == w
@@ -327,7 +377,7 @@ __global__ __launch_bounds__(64 * KWMAX) void qgemm_kernel(QgemmArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int t = 0; t < NW; t++) red[(((wave * MT + mt) * 4 + r) * NW + t) * kWave + lane] = acc[mt][t][r];
+                for (int t = 0; t < NW; t++) red[wave * LW + ((mt * 4 + r) * NW + t) * kWave + lane] = acc[mt][t][r];
         __syncthreads();
     }
     const QSeg& S = pick(a, si);
@@ -343,7 +393,7 @@ __global__ __launch_bounds__(64 * KWMAX) void qgemm_kernel(QgemmArgs a) {
             for (int t = 0; t < NW; t++) {
                 if (KWMAX > 1) {
                     float sum = 0.0f;
-                    for (int w = 0; w < KW; w++) sum += red[(((w * MT + mt) * 4 + r) * NW + t) * kWave + lane];
+                    for (int w = 0; w < KW; w++) sum += red[w * LW + ((mt * 4 + r) * NW + t) * kWave + lane];
                     v[t] = sum;
                 } else {
                     v[t] = acc[mt][t][r];
@@ -821,8 +871,8 @@ hipError_t launch_k(hipStream_t st, const QgemmArgs& a, int kw_in = 0) {
     const int mtt = (a.M + 15) / 16, gy = mtt / MT;
     const int G = a.K / 64;
     const int kw = kw_in > 0 ? min(KWMAX, kw_in) : (GPW == 0 ? KWMAX : min(KWMAX, (G + GPW - 1) / GPW));
-    const size_t lds = KWMAX > 1 ? sizeof(float) * (size_t)kw * MT * 4 * NW * kWave : 0;
-    hipLaunchKernelGGL((qgemm_kernel<MT, NW, GPW, KWMAX, EPI>), dim3(grid, gy), dim3(64 * kw), lds, st, a);
+    static_assert(KWMAX * wave_lds<MT, NW>() <= 64 * 1024, "the waves' LDS fits");
+    hipLaunchKernelGGL((qgemm_kernel<MT, NW, KWMAX, EPI>), dim3(grid, gy), dim3(64 * kw), (size_t)kw * (wave_lds<MT, NW>()), st, a);
     return hipGetLastError();
 }
 
