@@ -126,6 +126,37 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float* __restrict__ cs,
     gst(cs + 2 * k + 1, sinf(th));
 }
 
+// A page's K and V operands (64 x 64 bf16 each, 8 KB contiguous): loaded as they lie (1 KB a load:
+// one of 16 rows in the operand's order takes the address unit four times as long) and turned
+// round in 8 KB of the wave's own LDS, 16-byte chunks permuted by the row against bank conflicts.
+// ka[t][h]: row 32 (t / 2) + 8 (c / 4) + 4 (t % 2) + c % 4, chunk 2 j + h; va[dt][u]: dim 16 dt + c,
+// positions 32 u + 8 j + 0 .. 7.
+__device__ __forceinline__ void page_operands(const uint16_t* kb, const uint16_t* vb, uint4* lds, uint4 (&ka)[4][2],
+                                              uint4 (&va)[4][2]) {
+    const int lane = threadIdx.x % kWave, c = lane % 16, j = lane / 16;
+    auto kkey = [](int row) { return (row >> 1 & 1) | (row >> 3 & 3) << 1; };  // of 16 lanes' rows: 8 values, twice
+    auto vkey = [](int row) { return row >> 1 & 7; };
+    uint4 kr[8], vr[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) kr[i] = ldg4(kb + 512 * i + 8 * lane);
+#pragma unroll
+    for (int i = 0; i < 8; i++) vr[i] = ldg4(vb + 512 * i + 8 * lane);
+#pragma unroll
+    for (int i = 0; i < 8; i++) lds[8 * (8 * i + lane / 8) + (lane % 8 ^ kkey(8 * i + lane / 8))] = kr[i];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int row = 32 * (t / 2) + 8 * (c / 4) + 4 * (t % 2) + c % 4;
+#pragma unroll
+        for (int h = 0; h < 2; h++) ka[t][h] = lds[8 * row + ((2 * j + h) ^ kkey(row))];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) lds[8 * (8 * i + lane / 8) + (lane % 8 ^ vkey(8 * i + lane / 8))] = vr[i];
+#pragma unroll
+    for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) va[dt][u] = lds[8 * (16 * dt + c) + ((4 * u + j) ^ vkey(16 * dt + c))];
+}
+
 // ---- paged attention ------------------------------------------------------------------
 // Workgroup (split s, kv head g, sequence b); wave w takes page 4s + w (64
 // positions).  Both products run on the matrix cores with the kv head's grp
@@ -140,6 +171,7 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float* __restrict__ cs,
 //   bf16 hi + bf16 lo (two MFMAs), which keeps p to ~2^-17 relative.
 // The four waves' (max, sum, o) are combined through LDS into one partial.
 __global__ __launch_bounds__(256) void paged_attn_kernel(PagedAttnArgs a) {
+    __shared__ uint4 turn[4][512];
     __shared__ float so[3][16][64];
     __shared__ float sm[4][16], sl[4][16];
     const int s = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
@@ -170,17 +202,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(PagedAttnArgs a) {
         const uint16_t* kb = a.kp + pbase;
         const uint16_t* vb = a.vp + pbase;
         uint4 ka[4][2], va[4][2];
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int p = 32 * (t / 2) + 8 * (c / 4) + 4 * (t % 2) + c % 4;
-            const uint16_t* kr = kb + p * 64 + 16 * j;
-            ka[t][0] = ldg4(kr);
-            ka[t][1] = ldg4(kr + 8);
-        }
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++)
-#pragma unroll
-            for (int u = 0; u < 2; u++) va[dt][u] = ldg4(vb + (16 * dt + c) * 64 + 32 * u + 8 * j);
+        page_operands(kb, vb, turn[wave], ka, va);
         uint4 q[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
         if (c < a.grp) {
             const uint16_t* qr = a.qkv + (size_t)b * a.ldq + (g * a.grp + c) * 64 + 16 * j;
@@ -293,7 +315,7 @@ __global__ __launch_bounds__(256) void paged_attn_kernel(PagedAttnArgs a) {
 // took 65 us a layer one row at a time (1024 workgroups' K and V reads and 9 of 16 columns idle).
 __global__ __launch_bounds__(256) void prefill_attn_kernel(PagedAttnArgs a, int n, int hper) {
     extern __shared__ uint4 qs[];  // [16 rows][hper * 8 + 1]: scaled q
-    __shared__ float so[2][4][16][64];
+    __shared__ __align__(16) float so[2][4][16][64];
     __shared__ float sm[2][4][16], sl[2][4][16];
     const int s = blockIdx.x, hparts = (a.grp + hper - 1) / hper, g = blockIdx.y / hparts, h0 = blockIdx.y % hparts * hper,
               h1 = min(h0 + hper, a.grp), r0 = blockIdx.z * 16;
@@ -320,16 +342,7 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(PagedAttnArgs a, int 
         const size_t pbase = ((size_t)page * a.kvh + g) * 64 * 64;
         const uint16_t* kb = a.kp + pbase;
         const uint16_t* vb = a.vp + pbase;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int p = 32 * (t / 2) + 8 * (c / 4) + 4 * (t % 2) + c % 4;
-            ka[t][0] = ldg4(kb + p * 64 + 16 * j);
-            ka[t][1] = ldg4(kb + p * 64 + 16 * j + 8);
-        }
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++)
-#pragma unroll
-            for (int u = 0; u < 2; u++) va[dt][u] = ldg4(vb + (16 * dt + c) * 64 + 32 * u + 8 * j);
+        page_operands(kb, vb, reinterpret_cast<uint4*>(so) + 512 * wave, ka, va);  // before the barrier: so is free
     }
     const int qc = (h1 - h0) * 8, qld = hper * 8 + 1;
     for (int k = tid; k < 16 * qc; k += 256) {
