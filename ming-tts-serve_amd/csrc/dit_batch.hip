@@ -398,8 +398,8 @@ constexpr int k_slices(int K) {
 // launches a block (split-K partials and their reduce, the norm and the attention between the
 // GEMMs: 52 and 70 us a block) and a stage loop with two barriers per 128 k; these kernels take
 // the norm into the GEMM that reads it, the attention into the q/k/v GEMM, and keep the K slices
-// of a sum in the waves of one workgroup: 33 and 47 us a block, ten steps 4270 -> 2930 us (13
-// sequences) and 5720 -> 3850 us (64).  The rounding points and the order of every sum are the
+// of a sum in the waves of one workgroup: 33 and 45 us a block, ten steps 4270 -> 2930 us (13
+// sequences) and 5720 -> 3780 us (64).  The rounding points and the order of every sum are the
 // general path's.  What bounds them now: the redundant norm (each column block normalises its
 // rows: 3.4 of ff1's 7.8 us at 78 rows, 4.5 of 12.8 at 384), then the weight stream.
 //
@@ -654,21 +654,21 @@ struct FlowNorm {
     uint16_t *y_out, *y_steps;
 };
 
-// Norm + linear over 16 MT rows x 64 NT columns, 4 waves of NT column tiles each: ff1 with gelu
+// Norm + linear over 16 MT rows x 16 NT W columns, W waves of NT column tiles each: ff1 with gelu
 // (DE_GELU) and the final layer with CFG + Euler (DE_CFM).
-template <int D, int E, int MT, int NT>
-__global__ __launch_bounds__(256, 1) void flow_norm_kernel(FlowNorm a) {
+template <int D, int E, int MT, int NT, int W>
+__global__ __launch_bounds__(64 * W, 1) void flow_norm_kernel(FlowNorm a) {
     constexpr int S = D / 32, VS = E == DE_GELU ? k_slices(D) : 1, CH = NT > 1 ? 4 : 8;
     __shared__ uint4 As[MT * S * 64];
-    __shared__ uint4 Ws[4 * WStream<NT, CH>::kLds];
+    __shared__ uint4 Ws[W * WStream<NT, CH>::kLds];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, c = lane % 16,
               j = lane / 16;
     int bx, by;
     col_row(blockIdx.x, a.rb, bx, by);
-    const int r0 = 16 * MT * by, n0 = 64 * NT * bx;
+    const int r0 = 16 * MT * by, n0 = 16 * W * NT * bx;
     if (n0 >= a.N) return;
-    NormRows<D, MT, 4> rows;
-    rows.load(rows.v, a.x, wave, r0, a.R, a.gather);
+    NormRows<D, MT, W> rows;
+    if (wave < 4 * MT) rows.load(rows.v, a.x, wave, r0, a.R, a.gather);
     WStream<NT, CH> w;
     w.init(Ws + wave * w.kLds);
     float bias[NT];
@@ -728,20 +728,20 @@ __global__ __launch_bounds__(256, 1) void flow_norm_kernel(FlowNorm a) {
             }
     } else {
         lds_sync();
-        uint16_t* tile = reinterpret_cast<uint16_t*>(As);  // [MT][2 NT][lane][8]: the output in operand order
+        uint16_t* tile = reinterpret_cast<uint16_t*>(As);  // [MT][W NT / 2][lane][8]: the output in operand order
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
                 for (int t = 0; t < NT; t++)
-                    tile[frag_pos(16 * mt + 4 * j + r, 16 * (NT * wave + t) + c, 64 * NT)] =
+                    tile[frag_pos(16 * mt + 4 * j + r, 16 * (NT * wave + t) + c, 16 * W * NT)] =
                         f2bf((VS > 1 ? tot[mt][t][r] : acc[mt][t][r]) + bias[t]);
         lds_sync();
         // gelu on 8 values a turn, the tanh table's loads in one go (not one round trip a value)
 #pragma unroll 1
-        for (int q = threadIdx.x; q < MT * NT * 128; q += 256) {
-            const int rt = r0 / 16 + q / (128 * NT);
+        for (int q = threadIdx.x; q < MT * NT * W * 32; q += 64 * W) {
+            const int rt = r0 / 16 + q / (32 * W * NT);
             if (16 * rt >= a.R) break;
             const uint4 p = As[q];
             const uint32_t e[4] = {p.x, p.y, p.z, p.w};
@@ -757,7 +757,7 @@ __global__ __launch_bounds__(256, 1) void flow_norm_kernel(FlowNorm a) {
             for (int i = 0; i < 4; i++)
                 o[i] = pack_bf2(gelu_end(x[2 * i], tanh_bf16_of(th[2 * i], u[2 * i])),
                                 gelu_end(x[2 * i + 1], tanh_bf16_of(th[2 * i + 1], u[2 * i + 1])));
-            gst(reinterpret_cast<uint4*>(a.out) + ((size_t)rt * (a.N / 32) + n0 / 32) * 64 + q % (128 * NT),
+            gst(reinterpret_cast<uint4*>(a.out) + ((size_t)rt * (a.N / 32) + n0 / 32) * 64 + q % (32 * W * NT),
                 make_uint4(o[0], o[1], o[2], o[3]));
         }
     }
@@ -909,8 +909,10 @@ constexpr int kCus = 256;
 
 int xcd_grid(int cb, int rb) { return (cb + 7) / 8 * 8 * rb; }
 
-// Row and column tiles of a workgroup: the smallest of the list with at most one workgroup a CU
-// (a second one on some CUs doubles the launch's time; larger tiles than needed leave CUs idle).
+// Row and column tiles of a workgroup (columns in units; ff1's second one is four more waves, which
+// cover each other's norm and loads: 384 rows 14.5 -> 13.6 us against two tiles a wave): the
+// smallest of the list with at most one workgroup a CU (a second one on some CUs doubles the
+// launch's time; larger tiles than needed leave CUs idle).
 template <class F>
 hipError_t pick_tile(int R, int N, int unit, F launch) {
     const int rt = (R + 15) / 16;
@@ -928,12 +930,12 @@ template <int D>
 hipError_t launch_flow_ff1(hipStream_t st, FlowNorm a) {
     return pick_tile(a.R, a.N, 64, [&](int i, int rb, int grid) {
         a.rb = rb;
-        void (*k)(FlowNorm) = i == 0   ? flow_norm_kernel<D, DE_GELU, 1, 1>
-                              : i == 1 ? flow_norm_kernel<D, DE_GELU, 2, 1>
-                              : i == 2 ? flow_norm_kernel<D, DE_GELU, 3, 1>
-                              : i == 3 ? flow_norm_kernel<D, DE_GELU, 2, 2>
-                                       : flow_norm_kernel<D, DE_GELU, 3, 2>;
-        hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, a);
+        void (*k)(FlowNorm) = i == 0   ? flow_norm_kernel<D, DE_GELU, 1, 1, 4>
+                              : i == 1 ? flow_norm_kernel<D, DE_GELU, 2, 1, 4>
+                              : i == 2 ? flow_norm_kernel<D, DE_GELU, 3, 1, 4>
+                              : i == 3 ? flow_norm_kernel<D, DE_GELU, 2, 1, 8>
+                                       : flow_norm_kernel<D, DE_GELU, 3, 1, 8>;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(i < 3 ? 256 : 512), 0, st, a);
         return hipGetLastError();
     });
 }
@@ -1156,7 +1158,7 @@ hipError_t launch_flow_final(hipStream_t st, const uint16_t* h, int n, int D, co
                              uint16_t* y_out, uint16_t* y_steps) {
     const int rb = (2 * n + 15) / 16;
     const FlowNorm f{h, 2 * n, latent, rb, 3, norm, wf, bf, eps, nullptr, y, dt, sq, sde, step, steps, cfg, shift, y_out, y_steps};
-    void (*k)(FlowNorm) = D == 512 ? flow_norm_kernel<512, DE_CFM, 1, 1> : flow_norm_kernel<1024, DE_CFM, 1, 1>;
+    void (*k)(FlowNorm) = D == 512 ? flow_norm_kernel<512, DE_CFM, 1, 1, 4> : flow_norm_kernel<1024, DE_CFM, 1, 1, 4>;
     hipLaunchKernelGGL(k, dim3(xcd_grid(latent / 64, rb)), dim3(256), 0, st, f);
     return hipGetLastError();
 }

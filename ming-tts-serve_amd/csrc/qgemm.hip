@@ -17,11 +17,11 @@
 // l % 16, the same k-block; C[r] is (row 4 (l / 16) + r, column l % 16).
 // Here rows are activation rows (M), columns weight rows (N).  Within a group
 // (8 words) lane l takes words 2j and 2j+1 (j = l / 16), one per MFMA, so each
-// MFMA's 32 k lie in one group and a lane loads 8 contiguous bytes per row.
+// MFMA's 32 k lie in one group (the loads are by quads of lanes, see PairIn).
 //
 // Workgroup (column block x, row-tile group y): KW waves split the groups of
-// K; each wave accumulates MT x 16 rows by NW x 16 columns, with two groups'
-// loads in flight while one group's MFMAs run; the waves' partial sums are
+// K; each wave accumulates MT x 16 rows by NW x 16 columns, two groups at a
+// time with the next four groups' loads in flight; the waves' partial sums are
 // added through LDS and every wave applies the epilogue (QEpi) to its share of
 // the rows.  One call may concatenate up to three matrices along N (q/k/v;
 // gate/up), each a run of workgroups.  Staged activations are group-major:
@@ -1255,10 +1255,9 @@ bool launch_wide(hipStream_t st, QgemmArgs a, hipError_t& err) {
 }  // namespace
 
 // a.blocks is filled here.  Shapes: the LM head 4 column tiles x 2 row tiles
-// per wave, one wave per workgroup streaming all of K through the register
-// ring; gate/up 2 + 2 column tiles x 2 row tiles, two waves splitting K; q/k/v
-// one head (4 tiles) x 1 row tile, K in chunks of 2 groups over up to 8
-// waves; the narrow o/down projections 1 x 1, K in chunks of 5 groups over up
+// per wave, one wave per workgroup streaming all of K; gate/up 2 + 2 column tiles x 2 row tiles, two waves splitting K; q/k/v
+// one head (4 tiles) x 1 row tile, K in slices of 2 groups over up to 8
+// waves; the narrow o/down projections 1 x 1, K in slices of 5 groups over up
 // to 16 waves, so that they still spread over the CUs.  (Four row tiles per
 // wave would keep the accumulators in AGPRs.)  More than 64 rows: LDS-tiled
 // 64 x 64 tiles, except the narrow o/down projections (residual epilogue),

@@ -461,3 +461,26 @@ def test_prefill_row_tiles_equal_row_by_row(ming, ctx, small, pos0, L):
     (h0, (k0, v0)), (h1, (k1, v1)) = outs
     assert torch.equal(h0, h1)
     assert np.array_equal(k0, k1) and np.array_equal(v0, v1)
+
+
+@pytest.mark.parametrize("inter", [2048, 2240])
+def test_prefill_wide_chunks_of_k(ming, ctx, inter):
+    """The down projection of more than 64 rows with K from 2048 (LDS chunks of four groups, the last one ragged)
+    against that of 32-row chunks, bit for bit."""
+    S = syn_mod(ming)
+    spec = S.LmSpec(**dict(SMALL, inter=inter))
+    syn = S.SyntheticLm(ctx, spec, seed=23, quant=True, norm_std=0.1)
+    m, L = syn.model(), 77
+    x = ming.synth_normal_bf16(39, "prefill.wide.x", L * spec.hidden).reshape(L, spec.hidden)
+    xd = torch.from_numpy(x.view(np.int16)).cuda().view(torch.bfloat16)
+    outs = []
+    for rows in (128, 32):
+        bt = ming.LmBatch(m, rows, 128)
+        pk = S.PagedKv(spec, 1, 2, spare=1, seed=3)
+        hid = torch.empty((L, spec.hidden), dtype=torch.bfloat16, device="cuda")
+        bt.prefill(pk, one_row_table(pk), 0, x_in=xd, hidden=hid)
+        ctx.sync()
+        outs.append(hid)
+        bt.close()
+    m.close()
+    assert torch.equal(outs[0], outs[1])

@@ -107,3 +107,16 @@ def test_qgemm_shape_errors(ming, ctx):
     with pytest.raises(ming.MingError) as e:
         ctx.qgemm(dev_u16(x[:64]), wq, s, b, y)
     assert e.value.status == ming.MING_E_SHAPE
+
+
+@pytest.mark.parametrize("K,N", [(64, 16), (192, 80), (320, 130), (704, 64), (1088, 48)])
+@pytest.mark.parametrize("M", [3, 48])
+def test_qgemm_group_counts(ming, oracle, ctx, K, N, M):
+    """Odd numbers of groups of 64 (groups are taken two at a time; a wave's last may be one) and column counts that
+    end inside a tile of 16."""
+    x, wq, s, b = make(ming, ctx, K, N, M, seed=6)
+    L = oracle.Linear(wq.cpu().numpy().view(np.uint32), host_u16(s), host_u16(b))
+    yf = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    ctx.qgemm(dev_u16(x), wq, s, b, yf)
+    ctx.sync()
+    close_f32(yf.cpu().numpy(), oracle.linear_acc(L, x), f"qgemm f32 [{K}x{N}] M={M}")
