@@ -10,10 +10,9 @@
 // planes' sum are kept apart and added once, so the low planes' roundings fall
 // below the last bit.  4-bit weights enter as the exact values 16 + q (a nibble
 // OR-ed into bits 3..6 of bf16(16): two instructions a pair, where converting
-// q - 8 took five); each group of 64 is folded in f32 as s * sum (16 + q) x +
-// (b - 16 s) * sum x, the group sums of x coming from the same MFMAs against a
-// column of ones, and within a group the low planes are summed first, so only
-// the high plane's two MFMAs round at the sum's own size.
+// q - 8 took five); each group of 64 is folded in f32 from its sums with 16 + q
+// and of x itself (the same MFMAs against a column of ones), the high plane's and
+// the low planes' apart (q16_fold).
 //
 // Activations therefore travel between the kernels as planes, written by the
 // kernel that produces them in the MFMA A operand's order: bf16 [3][M / 16]
@@ -61,6 +60,16 @@ __device__ __forceinline__ uint4 unpack_q16(uint32_t w, uint32_t mask, uint32_t 
                       ((w >> 9) & mask) | magic);
 }
 constexpr uint32_t kQ16Mask = 0x00780078u, kQ16Magic = 0x41804180u;
+
+// acc + s sum q x + b sum x of one group from the sums with 16 + q (h: high plane, l: low planes)
+// and of x (xh, xl); off = b + 8 s.  sum (16 + q) x and 24 sum x are five times the size of their
+// difference sum (q - 8) x; the high plane's are sums of short mantissas (13 and 8 bits), all but
+// exact in f32, so the difference is taken plane by plane and rounds at its own size.  (Folding
+// s (h + l) + (b - 16 s) sum x instead left up to 1.2e-6 at 28 rows where the f32 MFMA path had 8e-7.)
+__device__ __forceinline__ float q16_fold(float s, float off, float h, float l, float xh, float xl, float acc) {
+    const float d = fmaf(-24.0f, xh, h) + fmaf(-24.0f, xl, l);
+    return fmaf(s, d, fmaf(off, xh + xl, acc));
+}
 
 // A value the compiler must keep in a register: mask and magic then make one v_and_or_b32
 // (which takes no literal operands).
@@ -331,8 +340,8 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
 #pragma unroll
             for (int k = 0; k < CH; k++) {
                 if (k >= n) break;
-                // the group sums of x, in every column's place
-                f32x4_t xs[MT];
+                // the group sums of x, in every column's place: the high plane's, and the low planes'
+                f32x4_t xh[MT], xl[MT];
                 uint4 x[2][NP][MT];
 #pragma unroll
                 for (int h = 0; h < 2; h++)
@@ -343,23 +352,26 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
                             x[h][p][mt] = NP == 1 ? pair_order(in.a[k][h][p][mt]) : in.a[k][h][p][mt];
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) {
-                    xs[mt] = kZero4;
+                    xl[mt] = kZero4;
 #pragma unroll
-                    for (int p = NP - 1; p >= 0; p--) xs[mt] = mma(x[1][p][mt], ones, mma(x[0][p][mt], ones, xs[mt]));
+                    for (int p = NP - 1; p > 0; p--) xl[mt] = mma(x[1][p][mt], ones, mma(x[0][p][mt], ones, xl[mt]));
+                    xh[mt] = mma(x[1][0][mt], ones, mma(x[0][0][mt], ones, kZero4));
                 }
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
                     const uint32_t* qr = q + (16 * t + c) * kQRow + 8 * k + j;
                     const uint4 b0 = unpack_q16(qr[0], mask, magic), b1 = unpack_q16(qr[4], mask, magic);
                     const float s = __uint_as_float(sc[64 * t + 16 * k + c]),
-                                off = fmaf(-16.0f, s, __uint_as_float(sc[64 * t + 32 + 16 * k + c]));
+                                off = fmaf(8.0f, s, __uint_as_float(sc[64 * t + 32 + 16 * k + c]));
 #pragma unroll
                     for (int mt = 0; mt < MT; mt++) {
-                        f32x4_t h = kZero4;
+                        f32x4_t l = kZero4;
 #pragma unroll
-                        for (int p = NP - 1; p >= 0; p--) h = mma(x[1][p][mt], b1, mma(x[0][p][mt], b0, h));
+                        for (int p = NP - 1; p > 0; p--) l = mma(x[1][p][mt], b1, mma(x[0][p][mt], b0, l));
+                        const f32x4_t h = mma(x[1][0][mt], b1, mma(x[0][0][mt], b0, kZero4));
 #pragma unroll
-                        for (int r = 0; r < 4; r++) hi[mt][t][r] = fmaf(s, h[r], fmaf(off, xs[mt][r], hi[mt][t][r]));
+                        for (int r = 0; r < 4; r++)
+                            hi[mt][t][r] = q16_fold(s, off, h[r], l[r], xh[mt][r], xl[mt][r], hi[mt][t][r]);
                     }
                 }
             }
@@ -511,7 +523,7 @@ __global__ __launch_bounds__(256, 2) void vtile_kernel(V3Gemm g) {
                 }
             if (sload) {
                 const float s = bf2f(r.s);
-                Ss[tid] = make_float2(s, fmaf(-16.0f, s, bf2f(r.b)));
+                Ss[tid] = make_float2(s, fmaf(8.0f, s, bf2f(r.b)));
             }
         } else {
 #pragma unroll
@@ -534,7 +546,7 @@ __global__ __launch_bounds__(256, 2) void vtile_kernel(V3Gemm g) {
     };
     auto compute = [&]() {
         if constexpr (WF == VW_Q4) {
-            f32x4_t th[MT][NT], xs[MT];
+            f32x4_t th[MT][NT], tl[MT][NT], xh[MT], xl[MT];  // high plane, low planes
             uint4 w[2][NT];
 #pragma unroll
             for (int h = 0; h < 2; h++)
@@ -547,10 +559,14 @@ __global__ __launch_bounds__(256, 2) void vtile_kernel(V3Gemm g) {
 #pragma unroll
                     for (int mt = 0; mt < MT; mt++) {
                         const uint4 a = afrag(p, mt, h);
-                        const bool first = p == 2 && h == 0;
-                        xs[mt] = mma(a, ones, first ? kZero4 : xs[mt]);
+                        const bool first = p != 1 && h == 0;
+                        f32x4_t& xs = p == 0 ? xh[mt] : xl[mt];
+                        xs = mma(a, ones, first ? kZero4 : xs);
 #pragma unroll
-                        for (int t = 0; t < NT; t++) th[mt][t] = mma(a, w[h][t], first ? kZero4 : th[mt][t]);
+                        for (int t = 0; t < NT; t++) {
+                            f32x4_t& acc = p == 0 ? th[mt][t] : tl[mt][t];
+                            acc = mma(a, w[h][t], first ? kZero4 : acc);
+                        }
                     }
 #pragma unroll
             for (int t = 0; t < NT; t++) {
@@ -559,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void vtile_kernel(V3Gemm g) {
                 for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        hi[mt][t][r] = fmaf(f.x, th[mt][t][r], fmaf(f.y, xs[mt][r], hi[mt][t][r]));
+                        hi[mt][t][r] = q16_fold(f.x, f.y, th[mt][t][r], tl[mt][t][r], xh[mt][r], xl[mt][r], hi[mt][t][r]);
             }
         } else {
 #pragma unroll
