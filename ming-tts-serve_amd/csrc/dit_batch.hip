@@ -15,6 +15,7 @@
 #include "args.h"
 #include "common.h"
 #include "dit_attn.h"
+#include "flow_steps.h"
 #include "internal.h"
 #include "tanh_tab.h"
 
@@ -386,11 +387,6 @@ __global__ __launch_bounds__(256) void dreduce_res_rms_kernel(DGemm a, const uin
             r4[p] = pack_bf2(bf_lo(we[p]) * rb(bf_lo(xv[k][p]) * inv), bf_hi(we[p]) * rb(bf_hi(xv[k][p]) * inv));
         gst(reinterpret_cast<uint4*>(hn + (size_t)m * N) + i, make_uint4(r4[0], r4[1], r4[2], r4[3]));
     }
-}
-
-// K slices of a sum for the bias, residual and gelu epilogues: a function of K alone.
-constexpr int k_slices(int K) {
-    return K >= 2048 && K % (4 * 64) == 0 ? 4 : (K >= 1024 && K % (2 * 64) == 0 ? 2 : 1);
 }
 
 // ---- the flow head's block in four launches -------------------------------------------------
@@ -774,7 +770,8 @@ struct FlowRes {
 // NT column tiles over 16 MT rows; the slices of a value meet in LDS and are added in slice order.
 template <int MT, int NT, int VS, int CW>
 __global__ __launch_bounds__(64 * VS * CW, 1) void flow_res_kernel(FlowRes a) {
-    constexpr int TH = 64 * VS * CW, CB = 16 * NT * CW, CH = MT * NT > 2 ? 4 : 8;
+    constexpr int TH = 64 * VS * CW, CB = 16 * NT * CW, CH = flow_set_steps(MT, NT);
+    static_assert(kFlowSetSteps % CH == 0, "flow_k_fits: whole register sets");
     constexpr int IT = (MT * 16 * CB / 4 + TH - 1) / TH;  // values (4 columns of a row) per thread at the end
     __shared__ __align__(16) float red[VS * CW * MT * 4 * NT * 64];
     __shared__ uint4 Ws[VS * CW * WStream<NT, CH>::kLds];
@@ -794,7 +791,7 @@ __global__ __launch_bounds__(64 * VS * CW, 1) void flow_res_kernel(FlowRes a) {
     for (int mt = 0; mt < MT; mt++)
         ap[mt] = a.a + ((size_t)min(r0 / 16 + mt, (a.R - 1) / 16) * (a.K / 32) + S * v) * 512 + 8 * lane;
     uint4 ar[2][CH][MT];
-    auto load = [&](int set, int s) {
+    auto load = [&](int set, int s) __attribute__((always_inline)) {
         w.load(set, s);
 #pragma unroll
         for (int k = 0; k < CH; k++)
@@ -806,7 +803,8 @@ __global__ __launch_bounds__(64 * VS * CW, 1) void flow_res_kernel(FlowRes a) {
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int t = 0; t < NT; t++) acc[mt][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    auto work = [&](int set) {
+    auto work = [&](int set) __attribute__((always_inline)) {
+        w.put(set);
 #pragma unroll
         for (int k = 0; k < CH; k++) {
             uint4 b[NT];
@@ -818,8 +816,7 @@ __global__ __launch_bounds__(64 * VS * CW, 1) void flow_res_kernel(FlowRes a) {
                 for (int t = 0; t < NT; t++) acc[mt][t] = mma(ar[set][k][mt], b[t], acc[mt][t]);
         }
     };
-    load(0, 0);
-    load(1, CH);
+    flow_first<CH>(S, load);
     // the epilogue's operands, in flight behind the first sets
     uint2 rv[IT], bv[IT];
 #pragma unroll
@@ -829,15 +826,7 @@ __global__ __launch_bounds__(64 * VS * CW, 1) void flow_res_kernel(FlowRes a) {
         rv[i] = make_uint2(gld(reinterpret_cast<const uint32_t*>(rp)), gld(reinterpret_cast<const uint32_t*>(rp) + 1));
         bv[i] = make_uint2(gld(bp) | (uint32_t)gld(bp + 1) << 16, gld(bp + 2) | (uint32_t)gld(bp + 3) << 16);
     }
-#pragma unroll 1
-    for (int s = 0; s < S; s += 2 * CH) {
-        w.put(0);
-        work(0);
-        if (s + 2 * CH < S) load(0, s + 2 * CH);
-        w.put(1);
-        work(1);
-        if (s + 3 * CH < S) load(1, s + 3 * CH);
-    }
+    flow_turns<CH>(S, load, work);
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -955,6 +944,7 @@ hipError_t launch_flow_res_vs(hipStream_t st, FlowRes a) {
 }
 
 hipError_t launch_flow_res(hipStream_t st, const FlowRes& a) {
+    if (!flow_k_fits(a.K)) return hipErrorInvalidValue;
     const int vs = k_slices(a.K);
     return vs == 4 ? launch_flow_res_vs<4, 1>(st, a) : (vs == 2 ? launch_flow_res_vs<2, 2>(st, a) : launch_flow_res_vs<1, 4>(st, a));
 }
@@ -1128,10 +1118,10 @@ hipError_t launch_cfm_final_batch(hipStream_t st, const uint16_t* h, int n, int 
 }
 
 // Shapes the four-launch block takes (launch_flow_block): heads of 64 over rows of three
-// positions, whole register sets of K per slice, and a normalised row of one or two 16-byte
-// chunks a lane.  Others run launch_dit_block_gemm.
+// positions, K slices of whole register sets (flow_k_fits), and a normalised row of one or two
+// 16-byte chunks a lane.  Others run launch_dit_block_gemm.
 bool flow_block_fits(int D, int F, int hd, int latent) {
-    return hd == 64 && (D == 512 || D == 1024) && F % 256 == 0 && (F / k_slices(F)) % 256 == 0 && latent % 64 == 0 &&
+    return hd == 64 && (D == 512 || D == 1024) && flow_k_fits(F) && latent % 64 == 0 &&
            k_slices(latent) == 1;
 }
 

@@ -197,7 +197,7 @@ def test_cfm_batch_row_tiles(ming, ctx, flowb, n):
                                              (768, 12, 1536)])
 def test_cfm_batch_shapes(ming, ctx, hidden, heads, ff):
     """Other shapes, bit for bit with the oracle in the batched kernels' order: the four-launch block (hidden 512 and
-    1024 with whole K slices of ff; one, two and four of them) and the general one (128, 768)."""
+    1024; one, two and four K slices of 512 values) and the general one (128, 768)."""
     S = syn_mod()
     spec = S.DitSpec(hidden=hidden, heads=heads, head_dim=64, ff=ff, cfm_blocks=2)
     syn = S.SyntheticFlow(ctx, spec, seed=67, norm_std=0.05, parts=("cfm",))
@@ -219,3 +219,36 @@ def test_cfm_batch_shapes(ming, ctx, hidden, heads, ff):
                     h = oracle.dit_block_fwd(ocfg(spec), blk, h, 2, 3, od.keep["cos"], od.keep["sin"])
                 assert_bits(g[b, i], oracle.cfm_final(od, h, 3, y_in, sde[b], i, 2.0, 0.25),
                             f"sequence {b} Euler step {i}")
+
+
+@pytest.mark.parametrize("hidden,heads", [(512, 8), (1024, 16)])
+@pytest.mark.parametrize("ff", [256, 768, 1536, 3072])
+def test_cfm_batch_odd_register_sets(ming, ctx, hidden, heads, ff):
+    """ff widths whose K slices are an odd number of 256-value register sets (one set, or three), at row counts on both
+    sides of every change of the tile (one to three row tiles by one or two column tiles): 64 sequences bit for bit with
+    the oracle, fewer with the first of the 64."""
+    S = syn_mod()
+    spec = S.DitSpec(hidden=hidden, heads=heads, head_dim=64, ff=ff, cfm_blocks=2)
+    syn = S.SyntheticFlow(ctx, spec, seed=68, norm_std=0.05, parts=("cfm",))
+    m = syn.cfm_model()
+    with oracle.dit_order(oracle.DIT_ORDER_DEVICE):
+        od = oracle_cfm(syn)
+    z, hist, noise, sde = inputs(ming, spec, 64, f"sets{hidden}.{ff}")
+    dev = [dev_u16(a) for a in (z, hist, noise, sde)]
+    steps = {}
+    for n in (64, 43, 42, 22, 21, 10, 1):
+        out = torch.empty((n, spec.latent), dtype=torch.bfloat16, device="cuda")
+        steps[n] = torch.empty((n, 10, spec.latent), dtype=torch.bfloat16, device="cuda")
+        m.sample_batch(n, *(d[:n] for d in dev), 2.0, 0.25, 1.0, out, steps[n])
+        ctx.sync()
+        assert torch.equal(out, steps[n][:, -1])
+        assert torch.equal(steps[n], steps[64][:n]), f"{n} sequences"
+    m.close()
+    g = host_u16(steps[64])
+    with oracle.dit_order(oracle.DIT_ORDER_MFMA):
+        for b, i in ((0, 0), (31, 4), (63, 9)):
+            y_in = noise[b] if i == 0 else g[b, i - 1]
+            h = oracle.cfm_rows(od, z[b], hist[b], y_in, i)
+            for blk in od.blocks:
+                h = oracle.dit_block_fwd(ocfg(spec), blk, h, 2, 3, od.keep["cos"], od.keep["sin"])
+            assert_bits(g[b, i], oracle.cfm_final(od, h, 3, y_in, sde[b], i, 2.0, 0.25), f"sequence {b} Euler step {i}")
