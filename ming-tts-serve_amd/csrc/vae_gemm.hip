@@ -8,11 +8,11 @@
 // a fifth of their cost (dense bf16 against f32: 1213 against 154 TFLOP/s for
 // a library product on this card).  The high plane's sum and the two low
 // planes' sum are kept apart and added once, so the low planes' roundings fall
-// below the last bit.  4-bit weights enter as the exact values 16 + q (a nibble
-// OR-ed into bits 3..6 of bf16(16): two instructions a pair, where converting
-// q - 8 took five); each group of 64 is folded in f32 from its sums with 16 + q
-// and of x itself (the same MFMAs against a column of ones), the high plane's and
-// the low planes' apart (q16_fold).
+// below the last bit.  4-bit weights enter as the exact values 2^-12 (16 + q) (a
+// nibble OR-ed into bits 3..6 of bf16(2^-8): two instructions a pair, where
+// converting q - 8 took five); each group of 64 is folded in f32 from its sums
+// with them and of 2^-12 x (the same MFMAs against a column of 2^-12), the high
+// plane's and the low planes' apart (q16_fold).
 //
 // Activations therefore travel between the kernels as planes, written by the
 // kernel that produces them in the MFMA A operand's order: bf16 [3][M / 16]
@@ -53,19 +53,23 @@ __device__ __forceinline__ void split3(float x, uint32_t (&p)[3]) {
 // The high halves of two words as a bf16 pair (lo in the low half).
 __device__ __forceinline__ uint32_t hi_pair(uint32_t lo, uint32_t hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
 
-// 8 nibbles of a packed word as the bf16 values 16 + q (exact) in pair order: nibble i and
-// i + 4 are one pair.
+// 8 nibbles of a packed word as the bf16 values 2^-12 (16 + q) (exact) in pair order: nibble i and
+// i + 4 are one pair.  The power of two keeps a group's sums finite for any finite x (64 values of
+// 2^-8 (1 + q / 16) < 2^-7, where 64 of 16 + q overflowed from 2^118 on) and changes no bit.
 __device__ __forceinline__ uint4 unpack_q16(uint32_t w, uint32_t mask, uint32_t magic) {
     return make_uint4(((w << 3) & mask) | magic, ((w >> 1) & mask) | magic, ((w >> 5) & mask) | magic,
                       ((w >> 9) & mask) | magic);
 }
-constexpr uint32_t kQ16Mask = 0x00780078u, kQ16Magic = 0x41804180u;
+constexpr uint32_t kQ16Mask = 0x00780078u, kQ16Magic = 0x3b803b80u, kQ16One = 0x39803980u;  // bf16(2^-12)
+constexpr float kQ16Scale = 4096.0f;  // what the sums lack (into the global scale: load_view)
 
-// acc + s sum q x + b sum x of one group from the sums with 16 + q (h: high plane, l: low planes)
-// and of x (xh, xl); off = b + 8 s.  sum (16 + q) x and 24 sum x are five times the size of their
-// difference sum (q - 8) x; the high plane's are sums of short mantissas (13 and 8 bits), all but
-// exact in f32, so the difference is taken plane by plane and rounds at its own size.  (Folding
-// s (h + l) + (b - 16 s) sum x instead left up to 1.2e-6 at 28 rows where the f32 MFMA path had 8e-7.)
+// acc + s sum q x + b sum x of one group, all over 2^12, from the sums with 2^-12 (16 + q) (h: high
+// plane, l: low planes) and of 2^-12 x (xh, xl); off = b + 8 s.  sum (16 + q) x and 24 sum x are five
+// times the size of their difference sum (q - 8) x; the high plane's are sums of short mantissas (13
+// and 8 bits), all but exact in f32, so the difference is taken plane by plane and rounds at its own
+// size.  (Folding s (h + l) + (b - 16 s) sum x instead left up to 1.2e-6 at 28 rows where the f32
+// MFMA path had 8e-7.)  An infinite x gives NaN where s q + b times it is infinite: the norm of the
+// row makes NaN of both.
 __device__ __forceinline__ float q16_fold(float s, float off, float h, float l, float xh, float xl, float acc) {
     const float d = fmaf(-24.0f, xh, h) + fmaf(-24.0f, xl, l);
     return fmaf(s, d, fmaf(off, xh + xl, acc));
@@ -105,7 +109,7 @@ struct V3View {
     const char *w, *wu;              // weights: the block's segment, up
     const uint16_t *s, *b, *su, *bu;  // affine scales and biases
     const uint16_t* bias;
-    float gs, gu;
+    float gs, gu;                    // global scales, times kQ16Scale for affine weights
     int n, start, rope;  // the segment's columns, its first column, rotary
     int M, K, ks, ldy, ldyp, ypair;
     const uint16_t* a;
@@ -169,7 +173,8 @@ __device__ __forceinline__ V3View<WF, EPI> load_view(const V3Gemm& g, int c0) {
         v.rope = s0.rope;
     }
     v.w = static_cast<const char*>(s0.w);
-    v.gs = s0.gs;
+    constexpr float kGs = WF == VW_Q4 ? kQ16Scale : 1.0f;
+    v.gs = kGs * s0.gs;
     v.n = s0.n;
     v.bias = s0.bias;
     v.s = s0.s;
@@ -178,7 +183,7 @@ __device__ __forceinline__ V3View<WF, EPI> load_view(const V3Gemm& g, int c0) {
         v.wu = static_cast<const char*>(s1.w);
         v.su = s1.s;
         v.bu = s1.b;
-        v.gu = s1.gs;
+        v.gu = kGs * s1.gs;
     }
     return v;
 }
@@ -325,7 +330,7 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
                             in.a[k][h][p][mt] =
                                 ldg4(at(v.a + p * v.aps + ((size_t)(u + k) * UH + h) * (NP == 1 ? 32 : 512), ao[mt]));
     };
-    const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+    const uint4 ones = make_uint4(kQ16One, kQ16One, kQ16One, kQ16One);
     const uint32_t mask = in_reg(kQ16Mask), magic = in_reg(kQ16Magic);
     auto work = [&](const V3Chunk<WF, NP, MT, NT>& in, int n) {  // n units
         if constexpr (WF == VW_Q4) {
@@ -538,7 +543,7 @@ __global__ __launch_bounds__(256, 2) void vtile_kernel(V3Gemm g) {
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int t = 0; t < NT; t++) hi[mt][t] = lo[mt][t] = kZero4;
-    const uint4 ones = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+    const uint4 ones = make_uint4(kQ16One, kQ16One, kQ16One, kQ16One);
     auto afrag = [&](int p, int mt, int h) { return As[((p * (BM / 16) + wm * MT + mt) * 2 + h) * 64 + lane]; };
     auto wfrag = [&](int t, int h) {
         const int k = 16 * (t * WN + wn) + c;

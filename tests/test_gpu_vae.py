@@ -151,3 +151,39 @@ def test_vae_latents_off_alignment(ming, ctx):
     ctx.sync()
     m.close()
     assert torch.equal(waves[0], waves[1])
+
+
+@pytest.mark.parametrize("T", [5, 17])
+def test_vae_4bit_large_values(ming, ctx, T):
+    """SwiGLU rows of about 2^122 (gate and up scaled by 2^61, down by 2^-115): a group's sums of them stay finite where
+    the dequantized weights' products do, on either side of 64 rows; the bars are those of check()."""
+    S = syn_mod()
+    syn = S.SyntheticVae(ctx, S.VaeSpec(**SMALL), seed=30, quant=True, std=0.05, norm_std=0.1)
+    for i in range(syn.spec.n_layers):
+        for name, e in (("gate_proj", 61), ("up_proj", 61), ("down_proj", -115)):
+            for k in "sb":
+                syn.tensors[f"audio.decoder.decoder.layers.{i}.mlp.{name}"][k].mul_(2.0 ** e)
+    check(ming, ctx, syn, T)
+
+
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("T", [9, 23])
+def test_vae_infinite_latent(ming, ctx, quant, T):
+    """A latent with an infinity makes NaN of exactly the samples that it does in the oracle (a row's norm turns an
+    infinite value into NaN), and the others keep their bars."""
+    S = syn_mod()
+    syn = S.SyntheticVae(ctx, S.VaeSpec(**dict(SMALL, window=4)), seed=31, quant=quant, std=0.05, norm_std=0.1)
+    om, spec = oracle_vae(syn), syn.spec
+    lat = ming.synth_normal_bf16(32, "vae.inf", T * spec.latent).reshape(T, spec.latent)
+    lat[3, 5] = 0x7f80
+    lat[4, 11] = 0xff80
+    wave = torch.empty(T * spec.patch * spec.hop, dtype=torch.float32, device="cuda")
+    m = syn.model(T)
+    m.decode(T, torch.from_numpy(lat.view(np.int16)).cuda().view(torch.bfloat16), wave)
+    ctx.sync()
+    m.close()
+    got, ref = wave.cpu().numpy(), oracle.vae_decode(om, lat)
+    bad = np.isnan(ref)
+    assert bad.any() and not bad.all()
+    assert np.array_equal(np.isnan(got), bad)
+    assert_close_f32(got[~bad], ref[~bad], "samples beside the infinite latents", 2e-4)
