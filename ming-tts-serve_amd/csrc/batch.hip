@@ -143,14 +143,17 @@ __device__ __forceinline__ void page_operands(const uint16_t* kb, const uint16_t
     for (int i = 0; i < 8; i++) vr[i] = ldg4(vb + 512 * i + 8 * lane);
 #pragma unroll
     for (int i = 0; i < 8; i++) lds[8 * (8 * i + lane / 8) + (lane % 8 ^ kkey(8 * i + lane / 8))] = kr[i];
+    wave_lds_order();
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const int row = 32 * (t / 2) + 8 * (c / 4) + 4 * (t % 2) + c % 4;
 #pragma unroll
         for (int h = 0; h < 2; h++) ka[t][h] = lds[8 * row + ((2 * j + h) ^ kkey(row))];
     }
+    wave_lds_order();
 #pragma unroll
     for (int i = 0; i < 8; i++) lds[8 * (8 * i + lane / 8) + (lane % 8 ^ vkey(8 * i + lane / 8))] = vr[i];
+    wave_lds_order();
 #pragma unroll
     for (int dt = 0; dt < 4; dt++)
 #pragma unroll

@@ -180,6 +180,11 @@ __device__ __forceinline__ void lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders a wave's own LDS accesses where lanes exchange values there: stores before it are seen by the other lanes'
+// loads after it, and loads before it read what was there before the stores after it.  The hardware runs a wave's LDS
+// accesses in order; the compiler knows only one lane's addresses and the types.
+__device__ __forceinline__ void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
+
 // Block-wide sum over blockDim.x threads (multiple of 64); `red` holds one
 // float per wave.  All threads get the result.
 __device__ __forceinline__ float block_sum(float v, float* red) {

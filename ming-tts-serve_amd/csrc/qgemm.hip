@@ -171,6 +171,7 @@ __device__ __forceinline__ void pair_mma(const PairIn<MT, NW>& p, int n, uint32_
     const int lane = threadIdx.x % kWave, c = lane % 16, j = lane / 16;
     uint32_t *q = lds, *sc = q + NW * 16 * kQRow;
     uint4* xl = reinterpret_cast<uint4*>(sc + NW * 64);  // [MT][16 rows][8 words], words permuted by the row
+    wave_lds_order();
 #pragma unroll
     for (int t = 0; t < NW; t++) {
         *reinterpret_cast<uint4*>(q + (16 * t + lane / 4) * kQRow + 4 * (lane % 4)) = p.w[t];
@@ -179,6 +180,7 @@ __device__ __forceinline__ void pair_mma(const PairIn<MT, NW>& p, int n, uint32_
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         if (k >= n) break;
+        if (k) wave_lds_order();
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
@@ -186,7 +188,7 @@ __device__ __forceinline__ void pair_mma(const PairIn<MT, NW>& p, int n, uint32_
                 const int row = 8 * h + lane / 8;
                 xl[128 * mt + 8 * row + (lane % 8 ^ row / 2)] = p.xa[k][mt][h];
             }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // other lanes' and types' values are read below
+        wave_lds_order();
         GroupIn<MT, NW> in;
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
@@ -372,6 +374,7 @@ __global__ __launch_bounds__(64 * KWMAX) void qgemm_kernel(QgemmArgs a) {
     }
     // the waves' partial sums through LDS; wave w then owns the row slots u = mt * 4 + r with u % KW == w
     if (KWMAX > 1) {
+        wave_lds_order();
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll

@@ -336,12 +336,13 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
         if constexpr (WF == VW_Q4) {
             uint32_t* q = reinterpret_cast<uint32_t*>(mine);  // [tile][16 rows][kQRow], [tile][s, s', b, b'][16]
             uint32_t* sc = q + NT * 16 * kQRow;
+            wave_lds_order();
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 *reinterpret_cast<uint4*>(q + (16 * t + lane / 4) * kQRow + 4 * (lane % 4)) = in.w[0][t];
                 sc[64 * t + lane] = (uint32_t)in.sb[t] << 16;
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the reads below are of other types and lanes
+            wave_lds_order();
 #pragma unroll
             for (int k = 0; k < CH; k++) {
                 if (k >= n) break;
@@ -389,6 +390,7 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
                 uint4 w[NT];
 #pragma unroll
                 for (int t = 0; t < NT; t++) wt[(k % 2 * NT + t) * 64 + 4 * (lane / 4) + (lane % 4 ^ lane / 16)] = in.w[k][t];
+                wave_lds_order();  // and the loads of step k - 1 before the stores of k + 1
 #pragma unroll
                 for (int t = 0; t < NT; t++) w[t] = wt[(k % 2 * NT + t) * 64 + 4 * c + (j ^ c / 4)];
 #pragma unroll
@@ -410,6 +412,7 @@ __global__ __launch_bounds__(64 * kSmallWaves<EPI>) void vsmall_kernel(V3Gemm g)
         load(u, in);
         work(in, u1 - u);
     }
+    wave_lds_order();
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
