@@ -463,6 +463,35 @@ def test_prefill_row_tiles_equal_row_by_row(ming, ctx, small, pos0, L):
     assert np.array_equal(k0, k1) and np.array_equal(v0, v1)
 
 
+@pytest.mark.parametrize("heads,kv,pos0,L", [
+    (14, 2, 0, 100), (14, 2, 10, 512), (14, 2, 700, 512), (14, 2, 1600, 512),  # 1, 2, 4 and 7 of 7 heads a workgroup
+    (8, 1, 3400, 512),                                                          # 8 of 8: the widest
+])
+def test_prefill_head_parts_equal_row_by_row(ming, ctx, heads, kv, pos0, L):
+    """How many of a kv head's heads share a workgroup of the prompt attention follows from the rows and the context
+    (the last part of seven is smaller): against chunks of 8 rows (one row a workgroup), bit for bit."""
+    S = syn_mod(ming)
+    spec = S.LmSpec(**dict(SMALL, hidden=64 * heads, heads=heads, kv_heads=kv, n_layers=1))
+    syn = S.SyntheticLm(ctx, spec, seed=24, quant=True, norm_std=0.1)
+    m, pages = syn.model(), (pos0 + L + 63) // 64
+    x = ming.synth_normal_bf16(40, "prefill.parts.x", L * spec.hidden).reshape(L, spec.hidden)
+    xd = torch.from_numpy(x.view(np.int16)).cuda().view(torch.bfloat16)
+    outs = []
+    for rows in (512, 8):
+        bt = ming.LmBatch(m, rows, 64 * pages)
+        pk = S.PagedKv(spec, 1, pages, spare=2, seed=8)
+        if pos0:
+            pk.fill_random([pos0], seed=41)
+        hid = torch.empty((L, spec.hidden), dtype=torch.bfloat16, device="cuda")
+        bt.prefill(pk, one_row_table(pk), pos0, x_in=xd, hidden=hid)
+        ctx.sync()
+        outs.append(hid)
+        bt.close()
+    m.close()
+    assert torch.equal(outs[0], outs[1])
+    assert torch.isfinite(outs[0].float()).all()
+
+
 @pytest.mark.parametrize("inter", [2048, 2240])
 def test_prefill_wide_chunks_of_k(ming, ctx, inter):
     """The down projection of more than 64 rows with K from 2048 (LDS chunks of four groups, the last one ragged)
