@@ -111,6 +111,13 @@ int ming_lm_batch_destroy(ming_lm_batch* b) {
     return MING_OK;
 }
 
+// Rows times cached positions from which a prompt's attention runs by 16-row tiles.  One row a workgroup reads rows *
+// positions, the tiles a sixteenth but in longer chains: a layer (14 heads on 2 kv heads) gains -0.6 .. +0.2 us at 64
+// rows to 512 positions, 80 to 272 and 128 to 128; +0.2 at 128 to 320, +0.4 at 64 to 1024, +0.7 at 32 to 2016, +0.1 at
+// 24 to 3924; +2.2 at 63 to 2047, +5.2 at 64 to 3964, +10.7 at 128 to 4028; 512 rows from 0 take 9.5 for 17 us, from
+// 1529 21.7 for 65.
+constexpr int64_t kTileReads = 40 * 1024;
+
 // One step of n_seq rows.  last >= 0: the rows are consecutive positions of one sequence, ending at last.
 static int batch_rows(ming_lm_batch* b, int32_t n_seq, const int32_t* tokens_dev, const void* x_in,
                       const ming_kv_pages* kv, const int32_t* page_table_dev, int32_t pages_per_seq, int32_t* pos_dev,
@@ -204,8 +211,9 @@ static int batch_rows(ming_lm_batch* b, int32_t n_seq, const int32_t* tokens_dev
         pa.grp = grp;
         pa.max_splits = max_splits;
         pa.scale = 0.125f;  // 1/sqrt(64)
-        // 19 rows: 4.7 us by 16-row tiles, 4.3 a row a workgroup; 512 rows from position 0: 9.5 and 17, from 1529: 21.7 and 65
-        e = last >= 0 && n_seq >= 64 ? launch_prefill_attn(st, pa, n_seq, last) : launch_paged_attn(st, pa, n_seq);
+        // a prompt's rows by 16-row tiles once one by one they would read 40 Ki cached positions of a kv head
+        e = last >= 0 && (int64_t)n_seq * (last + 1) >= kTileReads ? launch_prefill_attn(st, pa, n_seq, last)
+                                                                   : launch_paged_attn(st, pa, n_seq);
         if (e != hipSuccess) break;
         MergeArgs ma{pa.part, pos_dev, n_seq, c.heads, c.kv_heads, grp, max_splits, att, b->xs.p, xsum,
                      (n_seq + 15) / 16 * 16};

@@ -439,16 +439,17 @@ def test_prefill_capacity_error(ming, ctx, small):
     assert e.value.status == ming.MING_E_CTX_OVER_CAPACITY
 
 
-@pytest.mark.parametrize("pos0,L", [(0, 64), (0, 300), (40, 65), (199, 79), (250, 512)])
+@pytest.mark.parametrize("pos0,L", [(0, 64), (0, 300), (40, 65), (199, 79), (250, 512), (0, 203), (320, 97), (583, 64),
+                                    (1100, 37), (2400, 17), (3800, 11)])
 def test_prefill_row_tiles_equal_row_by_row(ming, ctx, small, pos0, L):
-    """The attention of 64 or more prompt rows (16-row tiles: ragged last tile, rows that end in different pages and
-    splits) against that of 32-row chunks (one row a workgroup), bit for bit."""
+    """A prompt's attention by 16-row tiles (from 40 Ki rows times positions: ragged last tile, rows that end in different
+    pages and splits) and short of that, against chunks of 8 rows (one row a workgroup), bit for bit."""
     S, spec, syn, m, _, _ = small
     pages = (pos0 + L + 63) // 64
     x = ming.synth_normal_bf16(37, "prefill.tiles.x", L * spec.hidden).reshape(L, spec.hidden)
     xd = torch.from_numpy(x.view(np.int16)).cuda().view(torch.bfloat16)
     outs = []
-    for rows in (512, 32):
+    for rows in (512, 8):
         bt = ming.LmBatch(m, rows, 64 * pages)
         pk = S.PagedKv(spec, 1, pages, spare=2, seed=7)
         if pos0:
