@@ -897,8 +897,6 @@ __global__ __launch_bounds__(256) void flow_rows_kernel(const uint16_t* __restri
     }
 }
 
-constexpr int kCus = 256;
-
 int xcd_grid(int cb, int rb) { return (cb + 7) / 8 * 8 * rb; }
 
 // Row and column tiles of a workgroup (columns in units; ff1's second one is four more waves, which
@@ -907,13 +905,13 @@ int xcd_grid(int cb, int rb) { return (cb + 7) / 8 * 8 * rb; }
 // launch's time; larger tiles than needed leave CUs idle).
 template <class F>
 hipError_t pick_tile(int R, int N, int unit, F launch) {
-    const int rt = (R + 15) / 16;
+    const int rt = (R + 15) / 16, cus = device_cus();
     const int cand[5][2] = {{1, 1}, {2, 1}, {3, 1}, {2, 2}, {3, 2}};
     for (int i = 0; i < 5; i++) {
         const int rb = (rt + cand[i][0] - 1) / cand[i][0], cb = (N + unit * cand[i][1] - 1) / (unit * cand[i][1]);
         if (N % (unit * cand[i][1])) continue;
         const int alt = i + 1 < 5 && N % (2 * unit) == 0;
-        if (rb * cb <= kCus || i == 4 || (i == 2 && !alt)) return launch(i, rb, xcd_grid(cb, rb));
+        if (rb * cb <= cus || i == 4 || (i == 2 && !alt)) return launch(i, rb, xcd_grid(cb, rb));
     }
     return hipErrorInvalidValue;
 }
@@ -957,7 +955,7 @@ hipError_t flow_block(hipStream_t st, const DitBlockDev& w, const uint16_t* x, i
                       const float* sin_t, uint16_t* att, uint16_t* x1, uint16_t* hh, uint16_t* out) {
     const int F = w.F, groups = R / 3, heads = D / 64;
     FlowQkv q{x, R, (groups + 4) / 5, w.norm1, {w.wq, w.wk, w.wv}, {w.bq, w.bk, w.bv}, w.eps, cos_t, sin_t, att};
-    if (q.rb * heads <= kCus) {
+    if (q.rb * heads <= device_cus()) {
         hipLaunchKernelGGL((flow_qkv_kernel<D, 1, 12>), dim3(xcd_grid(heads, q.rb)), dim3(768), 0, st, q);
     } else {
         q.rb = (groups + 9) / 10;

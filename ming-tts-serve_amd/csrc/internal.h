@@ -129,6 +129,7 @@ hipError_t launch_cfm_final_batch(hipStream_t st, const uint16_t* h, int n, int 
                                   const uint16_t* dt, const uint16_t* sq, const uint16_t* sde, int step, int steps,
                                   float cfg, float shift, uint16_t* hn, uint16_t* y_out, uint16_t* y_steps);
 
+int device_cus();
 bool flow_block_fits(int D, int F, int hd, int latent);
 hipError_t launch_flow_block(hipStream_t st, const DitBlockDev& w, const uint16_t* x, int R, const float* cos_t,
                              const float* sin_t, uint16_t* att, uint16_t* x1, uint16_t* hh, uint16_t* out);

@@ -26,11 +26,24 @@
 // the rows.  One call may concatenate up to three matrices along N (q/k/v;
 // gate/up), each a run of workgroups.  Staged activations are group-major:
 // xs [K/64][Mp][8] 16-byte words, xsum [K/64][Mp] (Mp = M rounded up to 16).
+#include <atomic>
+
 #include "batch.h"
 #include "common.h"
 #include "internal.h"
 
 namespace ming {
+
+// Compute units of the current device.
+int device_cus() {
+    static std::atomic<int> cus[64];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if ((n = cus[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
 
 namespace {
 
@@ -1151,18 +1164,6 @@ __global__ __launch_bounds__(64 * W) void qgemm_head_kernel(QgemmArgs a) {
     }
 }
 
-int head_grid() {
-    static int cus[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cus[dev]) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        cus[dev] = n;
-    }
-    return cus[dev];
-}
-
 // K = 896 (14 groups), whole units of 32 rows, scale and bias blocks 16-byte aligned
 bool head_fits(const QgemmArgs& a) {
     return a.nseg == 1 && a.M <= 64 && a.K == 896 && a.seg[0].N % 32 == 0 &&
@@ -1184,7 +1185,7 @@ hipError_t launch_head_g(hipStream_t st, QgemmArgs a) {
         if (e != hipSuccess) return e;
         raised[dev] = true;
     }
-    const int grid = min(head_grid(), (units + W - 1) / W);
+    const int grid = min(device_cus(), (units + W - 1) / W);
     hipLaunchKernelGGL((qgemm_head_kernel<MT, G, OUT, W, R>), dim3(grid), dim3(64 * W), lds, st, a);
     return hipGetLastError();
 }
