@@ -129,6 +129,17 @@ def test_vae_row_counts(ming, ctx, rows, quant, over):
     check(ming, ctx, syn, rows)
 
 
+@pytest.mark.parametrize("rows", [1, 17, 64, 65, 130])
+@pytest.mark.parametrize("quant", [False, True])
+def test_vae_wide_rows(ming, ctx, rows, quant):
+    """Hidden 1152 (18 heads on 2): rows too wide for the row kernel's registers are written and read back for the norm,
+    on either side of the linears' 64 rows; the bars are those of check()."""
+    S = syn_mod()
+    spec = S.VaeSpec(**dict(SMALL, patch=1, hidden=1152, heads=18, kv_heads=2))
+    syn = S.SyntheticVae(ctx, spec, seed=33, quant=quant, norm_std=0.1)
+    check(ming, ctx, syn, rows)
+
+
 @pytest.mark.parametrize("hop", [1, 6, 35, 11, 13 * 5])
 def test_vae_transform_lengths(ming, ctx, hop):
     """ISTFT by FFT passes (n_fft / 2 = 2, 12, 70: every radix, an odd one last) and by the basis GEMM (a prime
