@@ -141,7 +141,10 @@ struct VSeg {
 
 // C [M][N] = A [M][K] x W^T in f32; the output columns are the segments'
 // columns one after another (N = sum of seg[i].n).
-constexpr int kV3SmallRows = 64;  // rows up to which the unstaged kernel runs
+// Rows up to which the unstaged kernel runs.  A decode of 24 layers (896, ff 4864) in us, this kernel / LDS tiles, 4-bit
+// and bf16: 4 rows 791 / 1821 and 1067 / 1675, 36 rows 1164 / 1898 and 1432 / 1736, 64 rows 1274 / 1940 and
+// 1510 / 1765.  The line could lie higher: 96 rows 1424 / 1985 and 1658 / 1770, 128 rows 1727 / 2012 and 1986 / 1791.
+constexpr int kV3SmallRows = 64;
 struct V3Gemm {
     // np = 3: bf16 planes whose sum is A, in operand order (vae_gemm.hip), rows padded to 16;
     // np = 1: bf16 [M][K]

@@ -239,6 +239,9 @@ __device__ __forceinline__ void v3_epi(const V3View<WF, EPI>& v, int row, const 
 // that are 32 further in the same head (QKV: rotary pairs meet in one lane).
 template <int WF>
 constexpr int kUnitK = WF == VW_Q4 ? 64 : 32;
+// 4-bit: the two groups of one load.  bf16: units whose loads are all issued together; a decode of 24 layers in us with
+// chunks of 1, 2, 4 and 8: 4 rows 945, 1063, 1067, 1308, 28 rows 1034, 1136, 1203, 2122, 64 rows 1223, 1394, 1510, 2778
+// (the longest ones spill; shorter ones split K over more waves, another order of the sum).
 template <int WF>
 constexpr int kSmallCh = WF == VW_Q4 ? 2 : 4;
 template <int EPI>
@@ -786,6 +789,10 @@ __global__ __launch_bounds__(1024) void vattn_gqa_kernel(const float* qkv, int M
     for (int k = 0; k < 3; k++) gst(y + k * aps, (uint16_t)(pl[k] >> 16));
 }
 
+// Column blocks (times K slices) from which a workgroup takes two row tiles.  A decode of 24 layers in us with two tiles
+// from 1, 128 and 256 blocks on: bf16, 20..32 rows 1259, 1203, 1297, 36..48 rows 1495, 1441, 1397, 64 rows 1566, 1510,
+// 1584; 4-bit, 28 rows 1007, 929, 928, 36 rows 1241, 1164, 1005, 64 rows 1354, 1274, 1196 (there one tile each is better
+// at every row count: 256 and never measure the same).
 constexpr int kSmallTwoTiles = 128;
 
 template <int WF, int EPI, int NP>
