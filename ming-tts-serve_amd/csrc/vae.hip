@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void vola_kernel(const float* fr, int F, int n
     wave[i] = acc / fmaxf(env, 1e-11f);
 }
 
-// bf16 -> f32 (exact), for the latents fed to the f32 GEMM.
+// bf16 -> f32 (exact): a checkpoint's bf16 window, which the inverse transform reads as f32.
 __global__ __launch_bounds__(256) void vwiden_kernel(const uint16_t* x, int64_t n, float* y) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) y[i] = bf2f(x[i]);
