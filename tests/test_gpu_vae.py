@@ -149,6 +149,16 @@ def test_vae_transform_lengths(ming, ctx, hop):
     check(ming, ctx, syn, 5)
 
 
+@pytest.mark.parametrize("hop", [2048, 2058])
+def test_vae_longest_transforms(ming, ctx, hop):
+    """The longest transform that the FFT's LDS holds (4096 complex points, 64 KB) and the next one that factors (4116,
+    by the basis GEMM)."""
+    S = syn_mod()
+    syn = S.SyntheticVae(ctx, S.VaeSpec(**dict(SMALL, n_layers=1, patch=2, n_fft=4 * hop, hop=hop)), seed=34, std=0.05,
+                         norm_std=0.1)
+    check(ming, ctx, syn, 1)
+
+
 def test_vae_latents_off_alignment(ming, ctx):
     """Latents 2 bytes off a 16-byte boundary give the aligned call's bits."""
     S = syn_mod()
