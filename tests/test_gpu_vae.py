@@ -159,6 +159,21 @@ def test_vae_longest_transforms(ming, ctx, hop):
     check(ming, ctx, syn, 1)
 
 
+@pytest.mark.parametrize("four", [("fc1", "o_proj", "gate_proj", "up_proj"),
+                                  ("q_proj", "k_proj", "v_proj", "down_proj", "head.out")])
+@pytest.mark.parametrize("T", [9, 23])
+def test_vae_mixed_formats(ming, ctx, four, T):
+    """Some linears in 4 bits and the others in bf16, either way round: each kernel writes the planes in the order that
+    the next linear's format reads; on either side of 64 rows."""
+    S = syn_mod()
+    syn, bf = (S.SyntheticVae(ctx, S.VaeSpec(**SMALL), seed=35, quant=q, std=0.05, norm_std=0.1) for q in (True, False))
+    for name in syn.tensors:
+        if not name.endswith(four):
+            syn.tensors[name] = bf.tensors[name]
+    syn._build_views()
+    check(ming, ctx, syn, T)
+
+
 def test_vae_latents_off_alignment(ming, ctx):
     """Latents 2 bytes off a 16-byte boundary give the aligned call's bits."""
     S = syn_mod()
