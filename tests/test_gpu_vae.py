@@ -174,6 +174,23 @@ def test_vae_mixed_formats(ming, ctx, four, T):
     check(ming, ctx, syn, T)
 
 
+@pytest.mark.parametrize("T", [9, 23])
+def test_vae_global_scale(ming, ctx, T):
+    """A global scale of 1/4 with scales and biases four times as large is the same weight: the same bits, on either
+    side of 64 rows."""
+    S = syn_mod()
+    syn = S.SyntheticVae(ctx, S.VaeSpec(**SMALL), seed=36, quant=True, std=0.05, norm_std=0.1)
+    plain = run(ming, ctx, syn, T)
+    for v in syn.tensors.values():
+        if isinstance(v, dict):
+            v["s"].mul_(4.0)
+            v["b"].mul_(4.0)
+    syn.lin = lambda name: ming.linear(*(syn.tensors[name][k] for k in "wsb"), global_scale=0.25)
+    syn._build_views()
+    scaled = run(ming, ctx, syn, T)
+    assert all(np.array_equal(a, b) for a, b in zip(plain[1:], scaled[1:]))
+
+
 def test_vae_latents_off_alignment(ming, ctx):
     """Latents 2 bytes off a 16-byte boundary give the aligned call's bits."""
     S = syn_mod()
